@@ -187,6 +187,24 @@ int lock_workspace(DeviceState* ds, hipStream_t s, size_t bytes, WsLock& out,
   return HYPNO_HIP_OK;
 }
 
+// Whether stream s's workspace holds `bytes`, or may grow to: a stream under
+// graph capture cannot allocate, so there a call whose plain kernels need no
+// workspace takes those instead.
+bool workspace_can_hold(DeviceState* ds, hipStream_t s, size_t bytes) {
+  StreamWs* w = nullptr;
+  {
+    std::lock_guard<std::mutex> g(g_mu);
+    auto it = ds->workspaces.find(s);
+    if (it != ds->workspaces.end()) w = it->second.get();
+  }
+  if (w) {
+    std::lock_guard<std::mutex> g(w->mu);
+    if (w->buf.p && w->buf.cap >= bytes) return true;
+  }
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+}
+
 // [a, a + na) and [b, b + nb) share a byte (empty ranges share none).
 bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
   if (!a || !b || !na || !nb) return false;
@@ -217,6 +235,34 @@ struct FixedScratch {
   size_t bytes = 0;
   int cus = 256;
 };
+
+// Batches that no tuned kernel takes: the fp32-accurate block GEMM from 80M
+// products on, if its workspace can be had.  Below that one pass per token of
+// the any-length GEMV is as fast (Q4_0, N 2880, K 7200: 13.9 / 18.7 / 29.6 us
+// at 2 / 4 / 8 tokens against 20.3 / 20.3 / 20.7; N 512, K 1056, 8 tokens 4.6
+// against 14.3); the any-shape kernel beside it is slower from a few million.
+// *done says whether the block GEMM ran; otherwise the caller goes on.
+int try_block_gemm(int fmt, float* y, const uint8_t* w, size_t w_len, const float* x,
+                   const float* bias, size_t n, size_t m, size_t batch, hipStream_t s,
+                   DeviceState* ds, const FixedScratch* fixed, int cus, bool* done) {
+  const double from = gemv_any_ok(fmt, w, w_len, n, m) ? 80e6 : 4e6;
+  if (batch < 2 || (double)n * m * batch < from || !block_gemm_ok(fmt, w, w_len, n, m, batch))
+    return HYPNO_HIP_OK;
+  const BlockPlan p = block_plan(n, m, batch, cus);
+  const size_t bytes = block_gemm_workspace_bytes(p, n, m, batch);
+  if (fixed ? bytes > fixed->bytes : !workspace_can_hold(ds, s, bytes)) return HYPNO_HIP_OK;
+  WsLock ws;
+  if (fixed) {
+    ws.p = fixed->ptr;
+  } else {
+    int st = lock_workspace(ds, s, bytes, ws, "block GEMM workspace");
+    if (st) return st;
+  }
+  hipError_t e = launch_block_gemm(p, fmt, y, w, x, bias, n, m, batch, ws.p, s);
+  if (e != hipSuccess) return hip_fail(e, "block GEMM launch");
+  *done = true;
+  return HYPNO_HIP_OK;
+}
 
 int q4_0_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const float* bias,
              size_t n, size_t m, size_t batch, hipStream_t s,
@@ -272,13 +318,19 @@ int q4_0_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const flo
     if (e != hipSuccess) return hip_fail(e, "q4_0 skinny launch");
     return HYPNO_HIP_OK;
   }
-  if (batch >= kGemmMinBatch && !gemm_folded() && q4_0_gemm_exact_ok(w, w_len, n, m, batch)) {
-    WsLock ws;
-    st = scratch_for(q4_0_gemm_exact_workspace_bytes(batch, n, m, cus), ws, "GEMM workspace");
-    if (st) return st;
-    e = launch_q4_0_gemm_exact(y, w, x, bias, n, m, batch, ws.p, cus, s);
-    if (e != hipSuccess) return hip_fail(e, "q4_0 exact GEMM launch");
-    return HYPNO_HIP_OK;
+  // (the folded-scale kernels take K % 256 == 0 only; for other K the two
+  // numerics modes are one)
+  if (batch >= kGemmMinBatch && (!gemm_folded() || m % 256 != 0) &&
+      q4_0_gemm_exact_ok(w, w_len, n, m, batch)) {
+    const size_t bytes = q4_0_gemm_exact_workspace_bytes(batch, n, m, cus);
+    if (m % 256 == 0 || !fixed || bytes <= fixed->bytes) {
+      WsLock ws;
+      st = scratch_for(bytes, ws, "GEMM workspace");
+      if (st) return st;
+      e = launch_q4_0_gemm_exact(y, w, x, bias, n, m, batch, ws.p, cus, s);
+      if (e != hipSuccess) return hip_fail(e, "q4_0 exact GEMM launch");
+      return HYPNO_HIP_OK;
+    }
   }
   const bool v3 = batch >= kGemmMinBatch && q4_0_gemm_v3_ok(w, w_len, n, m, batch);
   if (v3 || (batch >= kGemmMinBatch && q4_0_gemm_ok(w, w_len, n, m, batch))) {
@@ -292,6 +344,9 @@ int q4_0_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const flo
     if (e != hipSuccess) return hip_fail(e, "q4_0 GEMM launch");
     return HYPNO_HIP_OK;
   }
+  bool done = false;
+  st = try_block_gemm(kFmtQ4_0, y, w, w_len, x, bias, n, m, batch, s, ds, fixed, cus, &done);
+  if (st || done) return st;
   if (q4_0_gemv_fast_ok(w, w_len, n, m) && aligned16(x)) {
     for (size_t t = 0; t < batch; t++) {
       e = launch_q4_0_gemv_fast(y + t * n, w, x + t * m, bias, n, m, cus, s);
@@ -299,7 +354,9 @@ int q4_0_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const flo
     }
     return HYPNO_HIP_OK;
   }
-  e = launch_q4_0_generic(y, w, w_len, x, bias, n, m, batch, s);
+  e = gemv_any_ok(kFmtQ4_0, w, w_len, n, m)
+          ? launch_gemv_any(kFmtQ4_0, y, w, w_len, x, bias, n, m, batch, s)
+          : launch_q4_0_generic(y, w, w_len, x, bias, n, m, batch, s);
   if (e != hipSuccess) return hip_fail(e, "q4_0 generic launch");
   return HYPNO_HIP_OK;
 }
@@ -351,6 +408,9 @@ int q8_0_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const flo
     }
     return HYPNO_HIP_OK;
   }
+  bool done = false;
+  st = try_block_gemm(kFmtQ8_0, y, w, w_len, x, bias, n, m, batch, s, ds, nullptr, cus, &done);
+  if (st || done) return st;
   if (q8_0_gemv_fast_ok(w, w_len, n, m) && aligned16(x)) {
     for (size_t t = 0; t < batch; t++) {
       e = launch_q8_0_gemv_fast(y + t * n, w, x + t * m, bias, n, m, cus, s);
@@ -358,7 +418,9 @@ int q8_0_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const flo
     }
     return HYPNO_HIP_OK;
   }
-  e = launch_q8_0_generic(y, w, x, bias, n, m, batch, s);
+  e = gemv_any_ok(kFmtQ8_0, w, w_len, n, m)
+          ? launch_gemv_any(kFmtQ8_0, y, w, w_len, x, bias, n, m, batch, s)
+          : launch_q8_0_generic(y, w, x, bias, n, m, batch, s);
   if (e != hipSuccess) return hip_fail(e, "q8_0 generic launch");
   return HYPNO_HIP_OK;
 }
@@ -1031,7 +1093,9 @@ int hypno_hip_q4_0_gemv_plan_run(const hypno_hip_gemv_plan* plan, void* stream) 
       e = launch_silu_mul(g.staged, d.x, g.pro.aux, d.m, s);
     if (e != hipSuccess) return hip_fail(e, "plan_run: prologue launch");
     if (g.staged) x = g.staged;
-    e = launch_q4_0_generic(d.y, d.w_q, d.w_len, x, d.bias, d.n, d.m, 1, s);
+    e = gemv_any_ok(kFmtQ4_0, d.w_q, d.w_len, d.n, d.m)
+            ? launch_gemv_any(kFmtQ4_0, d.y, d.w_q, d.w_len, x, d.bias, d.n, d.m, 1, s)
+            : launch_q4_0_generic(d.y, d.w_q, d.w_len, x, d.bias, d.n, d.m, 1, s);
     if (e != hipSuccess) return hip_fail(e, "plan_run: generic launch");
   }
   return HYPNO_HIP_OK;

@@ -97,6 +97,23 @@ __device__ __forceinline__ u32x4 unpack8(uint32_t q) {
   return r;
 }
 
+// Eight bytes -> eight exact fp16 values u - 128, in order (0x6400 | u is the
+// fp16 value 1024 + u).
+__device__ __forceinline__ u32x4 unpack8_bytes(uint32_t lo, uint32_t hi) {
+  const half2v off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+  u32x4 r;
+  r[0] = __builtin_amdgcn_perm(0x64646464u, lo, 0x04010400u);
+  r[1] = __builtin_amdgcn_perm(0x64646464u, lo, 0x04030402u);
+  r[2] = __builtin_amdgcn_perm(0x64646464u, hi, 0x04010400u);
+  r[3] = __builtin_amdgcn_perm(0x64646464u, hi, 0x04030402u);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const uint32_t u = r[i];
+    r[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, u) + off);
+  }
+  return r;
+}
+
 // Row r of X fp32 [M][K] -> row r of Xh fp16 [Mp][K], scaled by 2^sh with sh
 // chosen so that the row's largest |x| times 2^sh lies in [2^14, 2^15) (sh =
 // 0 for an all-zero row or one holding inf or NaN), and xexp[r] = -sh: the
@@ -210,6 +227,11 @@ hipError_t launch_dequantize_q4_0(float* out, const uint8_t* q, size_t n_blocks,
 hipError_t launch_q4_0_generic(float* y, const uint8_t* w, size_t w_len, const float* x,
                                const float* bias, size_t n, size_t m, size_t batch,
                                hipStream_t s);
+// One token (or `batch`, one by one), Q4_0 or Q8_0 (fmt: kFmt*), any
+// m % 32 == 0 up to 32768, w 4-byte aligned and full (gemv_any.hip).
+bool gemv_any_ok(int fmt, const uint8_t* w, size_t w_len, size_t n, size_t m);
+hipError_t launch_gemv_any(int fmt, float* y, const uint8_t* w, size_t w_len, const float* x,
+                           const float* bias, size_t n, size_t m, size_t batch, hipStream_t s);
 // Streaming decode GEMV for one token.  Requires m % 256 == 0 (m <= 15360),
 // lcm(m/64, 64) <= 1024, w 16-byte aligned, x 16-byte aligned,
 // w_len >= n*m/32*18.
@@ -344,7 +366,7 @@ hipError_t launch_q4_0_gemm_v3(float* y, const uint8_t* w, const float* x, const
 
 // MFMA prefill GEMM in the exact-nibble arithmetic (gemm_exact.hip): the
 // integer nibbles as fp16 into the matrix cores, each block's partial sum
-// scaled by its fp32 scale.  Requires m % 256 == 0, w 4-byte aligned, w_len
+// scaled by its fp32 scale.  Requires m % 64 == 0, w 4-byte aligned, w_len
 // full, W and the fp16 X under 4 GB.
 bool q4_0_gemm_exact_ok(const uint8_t* w, size_t w_len, size_t n, size_t m, size_t batch);
 size_t q4_0_gemm_exact_workspace_bytes(size_t batch, size_t n, size_t m, int num_cus);
@@ -359,6 +381,20 @@ size_t skinny_workspace_bytes(size_t batch, size_t n, size_t m, int num_cus);
 hipError_t launch_q4_0_skinny(float* y, const uint8_t* w, const float* x, const float* bias,
                               size_t n, size_t m, size_t batch, void* workspace, int num_cus,
                               hipStream_t s);
+
+// fp32-accurate batched GEMM for Q4_0 or Q8_0 weights (fmt: kFmt*) and any
+// K % 32 == 0 (gemm_block.hip).  `p` comes from block_plan for the same
+// arguments.
+struct BlockPlan {
+  int mt;      // 32-row tiles per wave
+  int splits;  // K pieces
+};
+bool block_gemm_ok(int fmt, const uint8_t* w, size_t w_len, size_t n, size_t m, size_t batch);
+BlockPlan block_plan(size_t n, size_t m, size_t batch, int num_cus);
+size_t block_gemm_workspace_bytes(const BlockPlan& p, size_t n, size_t m, size_t batch);
+hipError_t launch_block_gemm(const BlockPlan& p, int fmt, float* y, const uint8_t* w,
+                             const float* x, const float* bias, size_t n, size_t m, size_t batch,
+                             void* ws, hipStream_t s);
 
 // FP16 weights.
 hipError_t launch_f16_generic(float* y, const uint8_t* w, const float* x, const float* bias,

@@ -41,7 +41,7 @@
 //    writes an fp32 partial plane and split_k_reduce-style summation in
 //    split order finishes (fixed order: deterministic).
 //
-// Requirements (q4_0_gemm_exact_ok): K % 256 == 0, w 4-byte aligned and
+// Requirements (q4_0_gemm_exact_ok): K % 64 == 0 (whole stages), w 4-byte aligned and
 // holding N whole rows, W and the fp16 X under 4 GB (32-bit buffer offsets).
 #include <algorithm>
 
@@ -534,7 +534,7 @@ ExactPlan exact_plan(size_t batch, size_t n, size_t m, int num_cus) {
 }  // namespace
 
 bool q4_0_gemm_exact_ok(const uint8_t* w, size_t w_len, size_t n, size_t m, size_t batch) {
-  if (m == 0 || m % 256 != 0 || n == 0 || batch == 0) return false;
+  if (m == 0 || m % kEStageK != 0 || n == 0 || batch == 0) return false;
   if (((uintptr_t)w & 3) != 0) return false;
   if (n > (size_t)0x7FFFFFFF || m > (size_t)0x7FFFFFF || batch > (size_t)0x7FFFFFFF) return false;
   const size_t wbytes = n * (m / kBlockElems) * kBlockBytes;

@@ -1,0 +1,100 @@
+"""Q4_0 and Q8_0 products at row lengths that no tuned kernel takes: one token
+through the any-length GEMV, batches through the fp32-accurate block GEMM (and,
+for Q4_0 from 16 tokens at K % 64 == 0, the prefill GEMM).  The cases sit at
+the edges of their tiles: odd numbers of blocks per row (rows on 2-byte
+boundaries), buffers that end with the last row, x off a 16-byte boundary, one
+row or column past a tile, K pieces, lanes shared by several short rows."""
+import ctypes
+
+import numpy as np
+import pytest
+
+CASES = [  # dtype, tokens, n, m
+    (dt, tok, n, m)
+    for dt in ("q4_0", "q8_0")
+    for tok, n, m in [
+        # the any-length GEMV: 8, 16, 32 and 64 lanes per row
+        (1, 1, 32), (1, 33, 96), (1, 257, 288), (1, 31, 544), (1, 100, 1056), (1, 65, 11008),
+        (1, 7, 32768), (1, 5, 32800), (2, 97, 1120), (7, 513, 4128), (33, 257, 2080),
+        # the block GEMM: 32-, 64- and 128-row tiles, one row or column past them
+        (5, 4097, 4128), (16, 1300, 4128), (33, 1030, 2400), (64, 520, 2464), (65, 1290, 1120),
+        (129, 600, 1120), (300, 257, 1120),
+        # whole 64-column stages, from 16 tokens the prefill GEMM (Q4_0)
+        (16, 640, 2880), (17, 129, 4160)]
+]
+
+
+def _run(lib, torch, dt, wb, x, bias, n, m, tokens, shift):
+    buf = torch.empty(x.size + shift, dtype=torch.float32, device="cuda")
+    dx = buf[shift:]
+    dx.copy_(torch.from_numpy(x.ravel()))
+    dw = torch.from_numpy(wb).cuda()
+    db = torch.from_numpy(bias).cuda()
+    y = torch.full((tokens * n,), float("nan"), dtype=torch.float32, device="cuda")
+    fn = {"q4_0": lib.hypno_hip_matmul_q4_0_dev, "q8_0": lib.hypno_hip_matmul_q8_0_dev}[dt]
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    assert fn(p(y), p(dw), wb.size, p(dx), p(db), n, m, tokens, None) == 0
+    torch.cuda.synchronize()
+    return y.cpu().numpy().reshape(tokens, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("dt,tokens,n,m", CASES)
+def test_any_shape(orc, dt, tokens, n, m, shift):
+    import torch
+
+    from hypno_amd import _lib
+    print(f"{dt} tokens={tokens} n={n} m={m} shift={shift}", flush=True)
+    rng = np.random.default_rng(n * 7 + m + tokens)
+    w = (rng.standard_normal(n * m) * 0.02).astype(np.float32)
+    wb = orc.quantize_q4_0(w) if dt == "q4_0" else orc.quantize_q8_0(w)
+    x = rng.standard_normal((tokens, m)).astype(np.float32)
+    x[:, ::97] *= 30.0
+    bias = rng.standard_normal(n).astype(np.float32)
+    got = _run(_lib.load(), torch, dt, wb, x, bias, n, m, tokens, shift)
+    f64 = orc.matmul_q4_0_f64 if dt == "q4_0" else orc.matmul_q8_0_f64
+    ref = np.stack([f64(wb, x[t], bias, n, m) for t in range(tokens)])
+    # from 16 tokens whole 64-column stages round x to fp16 (relative 2^-12 at
+    # random, 3e-4 of the result at most here); everything else is fp32 sums,
+    # whose random error stays under sqrt(K) 2^-24 of the largest product sum
+    if tokens >= 16 and m % 64 == 0:
+        assert orc.rel_l2(got, ref) <= 2e-3
+    else:
+        for t in range(tokens):
+            assert orc.normwise_err(got[t], ref[t]) <= 2e-5, t
+
+
+@pytest.mark.gpu
+def test_any_shape_plan_and_capture(orc):
+    """A plan's job with K = 11008 (any-length GEMV), and a ragged batch
+    captured on a stream that has no workspace yet, replayed."""
+    import torch
+
+    import hypno_amd as hk
+    n, m, tokens = 320, 1120, 24
+    rng = np.random.default_rng(5)
+    wb = orc.quantize_q4_0((rng.standard_normal(n * 11008) * 0.02).astype(np.float32))
+    x = rng.standard_normal(11008).astype(np.float32)
+    dw, dx = torch.from_numpy(wb).cuda(), torch.from_numpy(x).cuda()
+    y = torch.full((n,), float("nan"), device="cuda")
+    plan = hk.GemvPlan([(y, dw, dx, None, n, 11008)])
+    plan.run()
+    torch.cuda.synchronize()
+    assert orc.normwise_err(y.cpu().numpy(), orc.matmul_q4_0_f64(wb, x, None, n, 11008)) <= 2e-5
+    wb = orc.quantize_q4_0((rng.standard_normal(n * m) * 0.02).astype(np.float32))
+    xb = rng.standard_normal((tokens, m)).astype(np.float32)
+    dw, dx = torch.from_numpy(wb).cuda(), torch.from_numpy(xb).cuda()
+    y = torch.zeros(tokens, n, device="cuda")
+    ref = np.stack([orc.matmul_q4_0_f64(wb, xb[t], None, n, m) for t in range(tokens)])
+    s = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        hk.batch_matmul(y, dw, hk.DType.Q4_0, dx, n, m, tokens)
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        for t in range(tokens):
+            assert orc.normwise_err(y[t].cpu().numpy(), ref[t]) <= 2e-5
