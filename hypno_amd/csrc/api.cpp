@@ -446,6 +446,31 @@ int q4_0_col_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const
     if (st) return st;
     cus = ds->cus;
   }
+  hipError_t e;
+  // Many tokens: the tensor expanded once to fp16 pairs and a GEMM, against
+  // the one-token kernel over groups of tokens.  Measured per call (us, old
+  // and new): 2048 x 2048 15.7 / 20.4 at 8 tokens, 42.7 / 22.8 at 32, 139 /
+  // 31.8 at 128; 5632 x 2048 19.5 / 31.5 at 4, 54.1 / 30.7 at 16, 399 / 40.6
+  // at 128; 14336 x 4096 104 / 106 at 16, 201 / 108 at 32; 512 x 544 16.8 /
+  // 17.0 at 64: about 5 us and 0.25 us per million weights and token (0.11
+  // beyond 32M, which fill the chip) against 15 us, 1.45 us per million
+  // weights and 0.025 per million and token.  Up to 512 MB of expansion.
+  {
+    const double mw = (double)n * m * 1e-6;
+    const double one = 5.0 + batch * mw * (mw < 32.0 ? 0.25 : 0.11);
+    const double many = 15.0 + mw * (1.45 + 0.025 * batch);
+    if (batch > 1 && many < one && mw <= 128.0 && q4_0_col_gemm_ok(w, w_len, n, m, batch)) {
+      const size_t bytes = q4_0_col_gemm_workspace_bytes(n, m, batch, cus);
+      if (workspace_can_hold(ds, s, bytes)) {
+        WsLock ws;
+        st = lock_workspace(ds, s, bytes, ws, "column-major workspace");
+        if (st) return st;
+        e = launch_q4_0_col_gemm(y, w, w_len, x, bias, n, m, batch, ws.p, cus, s);
+        if (e != hipSuccess) return hip_fail(e, "column-major GEMM launch");
+        return HYPNO_HIP_OK;
+      }
+    }
+  }
   // Tokens go in groups (one main and one reduction launch each) whose
   // partial planes fit 64 MB of workspace, at most 256 tokens a group.
   WsLock ws;
@@ -453,7 +478,6 @@ int q4_0_col_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const
   size_t group = batch < 256 ? batch : 256;
   if (per && group > 1 && per * group > ((size_t)64 << 20))
     group = ((size_t)64 << 20) / per > 1 ? ((size_t)64 << 20) / per : 1;
-  hipError_t e;
   if (per) {
     st = lock_workspace(ds, s, per * group, ws, "column-major workspace");
     if (st) return st;
@@ -505,6 +529,22 @@ int f16_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const floa
     e = launch_f16_gemm_v2(y, w, x, bias, n, m, batch, ws.p, cus, s);
     if (e != hipSuccess) return hip_fail(e, "f16 GEMM launch");
     return HYPNO_HIP_OK;
+  }
+  // Rows that are no multiple of the GEMMs' 64-column stages: the fp32-accurate
+  // pair GEMM, against one GEMV per token (us: 2880 x 7200 24.2 / 26.3 at 2
+  // tokens, 29.3 / 823 at 64; 4096 x 2080 12.7 / 12.6 at 2, 12.9 / 48.5 at 8;
+  // 1024 x 544 11.0 / 6.1 at 2, 12.9 / 23.4 at 8).
+  if (batch >= 2 && (batch >= 4 || (double)n * m * batch >= 17e6) &&
+      f16_pair_gemm_ok(w, n, m, batch)) {
+    const size_t bytes = f16_pair_gemm_workspace_bytes(n, m, batch, cus);
+    if (workspace_can_hold(ds, s, bytes)) {
+      WsLock ws;
+      st = lock_workspace(ds, s, bytes, ws, "GEMM workspace");
+      if (st) return st;
+      e = launch_f16_pair_gemm(y, w, x, bias, n, m, batch, ws.p, cus, s);
+      if (e != hipSuccess) return hip_fail(e, "f16 pair GEMM launch");
+      return HYPNO_HIP_OK;
+    }
   }
   if (f16_gemv_fast_ok(w, n, m) && aligned16(x)) {
     for (size_t t = 0; t < batch; t++) {

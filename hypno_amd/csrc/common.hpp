@@ -396,6 +396,29 @@ hipError_t launch_block_gemm(const BlockPlan& p, int fmt, float* y, const uint8_
                              const float* x, const float* bias, size_t n, size_t m, size_t batch,
                              void* ws, hipStream_t s);
 
+// X fp32 [batch][m] -> fp16 [batch][kp] hi parts and a plane of lo parts in
+// natural column order, per-row exponents at xexp; with `clear`, *clear = 0
+// and the exponent of a row holding inf or NaN is INT_MIN.
+hipError_t launch_x_hilo(void* xh, int* xexp, const float* x, size_t batch, size_t m, size_t kp,
+                         uint32_t* clear, hipStream_t s);
+// y[mn] = the sum of `splits` planes of mn floats in order (+ bias[i % n]).
+hipError_t launch_split_reduce(float* y, const float* part, const float* bias, size_t mn, size_t n,
+                               int splits, hipStream_t s);
+
+// fp32-accurate batched GEMMs on fp16 operand pairs (gemm_pair.hip):
+// column-major Q4_0 expanded once per call, and fp16 weights with any
+// m % 32 == 0.
+bool q4_0_col_gemm_ok(const uint8_t* w, size_t w_len, size_t n, size_t m, size_t batch);
+size_t q4_0_col_gemm_workspace_bytes(size_t n, size_t m, size_t batch, int num_cus);
+hipError_t launch_q4_0_col_gemm(float* y, const uint8_t* w, size_t w_len, const float* x,
+                                const float* bias, size_t n, size_t m, size_t batch, void* ws,
+                                int num_cus, hipStream_t s);
+bool f16_pair_gemm_ok(const uint8_t* w, size_t n, size_t m, size_t batch);
+size_t f16_pair_gemm_workspace_bytes(size_t n, size_t m, size_t batch, int num_cus);
+hipError_t launch_f16_pair_gemm(float* y, const uint8_t* w, const float* x, const float* bias,
+                                size_t n, size_t m, size_t batch, void* ws, int num_cus,
+                                hipStream_t s);
+
 // FP16 weights.
 hipError_t launch_f16_generic(float* y, const uint8_t* w, const float* x, const float* bias,
                               size_t n, size_t m, size_t batch, hipStream_t s);

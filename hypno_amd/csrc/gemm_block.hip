@@ -416,15 +416,17 @@ block_split_reduce_kernel(float* __restrict__ y, const float* __restrict__ part,
 // NaN), xexp[row] = -sh, columns K .. Kp - 1 zero.  kPerm writes each group
 // of 8 columns in the Q4_0 unpack order e0,e4,e1,e5,e2,e6,e3,e7.  The row is
 // read once if it fits the registers (K <= 16384 and 16-byte aligned), twice
-// otherwise.
+// otherwise.  With `clear`, *clear is set to 0 and the exponent of a row
+// holding inf or NaN to INT_MIN.
 constexpr int kXG = 8;
 template <bool kPerm>
 __global__ void __launch_bounds__(256)
 x_rows_block_kernel(u32x4* __restrict__ xh, int* __restrict__ xexp, const float* __restrict__ x,
-                    size_t plane, int K, int Kp) {
+                    size_t plane, int K, int Kp, uint32_t* __restrict__ clear) {
   __shared__ uint32_t red[4];
   const int row = blockIdx.x;
   const int t = threadIdx.x;
+  if (clear && row == 0 && t == 0) *clear = 0;
   const int groups = K / 8, gp = Kp / 8;
   u32x4* dst = xh + (size_t)row * gp;
   const float* src = x + (size_t)row * K;
@@ -480,7 +482,10 @@ x_rows_block_kernel(u32x4* __restrict__ xh, int* __restrict__ xexp, const float*
       const _Float16 h0 = (_Float16)s0, h1 = (_Float16)s1;
       a[j] = (uint32_t)__builtin_bit_cast(uint16_t, h0) |
              ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-      const _Float16 l0 = (_Float16)(s0 - (float)h0), l1 = (_Float16)(s1 - (float)h1);
+      // (inf - inf: the hi part alone carries an infinity)
+      const float r0 = s0 - (float)h0, r1 = s1 - (float)h1;
+      const _Float16 l0 = (_Float16)(r0 == r0 ? r0 : 0.0f);
+      const _Float16 l1 = (_Float16)(r1 == r1 ? r1 : 0.0f);
       b[j] = (uint32_t)__builtin_bit_cast(uint16_t, l0) |
              ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
     }
@@ -502,7 +507,7 @@ x_rows_block_kernel(u32x4* __restrict__ xh, int* __restrict__ xexp, const float*
     dst[groups + t] = u32x4{0u, 0u, 0u, 0u};
     dst[plane + groups + t] = u32x4{0u, 0u, 0u, 0u};
   }
-  if (t == 0) xexp[row] = -sh;
+  if (t == 0) xexp[row] = clear && mb >= 0x7F800000u ? (int)0x80000000u : -sh;
 }
 
 size_t rup(size_t v, size_t a) { return (v + a - 1) / a * a; }
@@ -605,7 +610,7 @@ hipError_t launch_block_gemm(const BlockPlan& p, int fmt, float* y, const uint8_
 
   auto conv = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)batch), dim3(256), 0, s, static_cast<u32x4*>(ws),
-                       xexp, x, batch * kp / 8, (int)m, (int)kp);
+                       xexp, x, batch * kp / 8, (int)m, (int)kp, nullptr);
     return hipGetLastError();
   };
   const bool q8 = fmt == kFmtQ8_0, odd = a.B % 2 != 0;
@@ -616,9 +621,20 @@ hipError_t launch_block_gemm(const BlockPlan& p, int fmt, float* y, const uint8_
   else
     e = odd ? launch_block_mt<kFmtQ4_0, true>(p, a, s) : launch_block_mt<kFmtQ4_0, false>(p, a, s);
   if (e != hipSuccess || p.splits == 1) return e;
-  const size_t mn = batch * n;
+  return launch_split_reduce(y, a.part, bias, batch * n, n, p.splits, s);
+}
+
+hipError_t launch_split_reduce(float* y, const float* part, const float* bias, size_t mn, size_t n,
+                               int splits, hipStream_t s) {
   hipLaunchKernelGGL(block_split_reduce_kernel, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0,
-                     s, y, a.part, bias, mn, (int)n, p.splits);
+                     s, y, part, bias, mn, (int)n, splits);
+  return hipGetLastError();
+}
+
+hipError_t launch_x_hilo(void* xh, int* xexp, const float* x, size_t batch, size_t m, size_t kp,
+                         uint32_t* clear, hipStream_t s) {
+  hipLaunchKernelGGL(x_rows_block_kernel<false>, dim3((unsigned)batch), dim3(256), 0, s,
+                     static_cast<u32x4*>(xh), xexp, x, batch * kp / 8, (int)m, (int)kp, clear);
   return hipGetLastError();
 }
 

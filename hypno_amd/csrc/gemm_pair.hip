@@ -1,0 +1,516 @@
+// fp32-accurate batched GEMM on fp16 operand pairs, for gfx950:
+// Y[M][N] = X[M][K] . W[N][K]^T (+ bias) with X = (xh + xl) 2^e per token and
+// W = wh (fp16 weights) or wh + wl, and its users: column-major Q4_0 batches
+// (kernels.rs:403-535, turbo.rs:322-326) and fp16 batches whose rows are no
+// multiple of 64.
+//
+// Column-major Q4_0: W_col[k][j] keeps 32 outputs j of one input k in a
+// block, so the scale d changes with k inside an output's sum and cannot be
+// applied to partial sums.  q4_0_col_expand_kernel turns the tensor once per
+// call into row-major fp16 pairs: wh = fp16(n d) rounded to nearest and wl =
+// n d - wh, which fp16 holds exactly (a 4-bit integer times an 11-bit d leaves
+// at most 4 units of d's last place, and that place is at least 2^-24).  The
+// GEMM then adds xh wh + xl wh + xh wl in fp32 on the matrix cores; what it
+// leaves out, xl wl, is 2^-24 of a product.
+//
+// What bounds it: at a few hundred tokens the expansion (4 bytes written per
+// weight) and its read back; the one-token kernel it stands in for reads the
+// weights once per token (128 tokens, 5632 x 2048: 399 us; this 41).
+//
+//  * Work-group = 8 waves on a 32 MT x 256 tile of Y, 32 columns a wave;
+//    32x32x16 MFMAs.  Lane (n, h) loads the 64 bytes of its column and lane
+//    half straight into registers, one stage of 64 K ahead.
+//  * X: hi rows then lo rows by DMA into a ring of four LDS stages, 16-byte
+//    chunk c of row r in slot c ^ ((r >> 1) & 7) (16 rows of an operand read
+//    hit distinct banks); one barrier per stage publishes the stage two ahead.
+#include <algorithm>
+
+#include "common.hpp"
+
+namespace hypno {
+
+namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+constexpr int kPWaves = 8;
+constexpr int kPThreads = 64 * kPWaves;
+constexpr int kPBN = 32 * kPWaves;
+constexpr int kPStageK = 64;
+constexpr int kPRowBytes = kPStageK * 2;
+constexpr int kPRing = 4;
+[[maybe_unused]] constexpr uint32_t kBigScale = 0x6FFF;  // fp16 bits of 8188: 8 * 8188 is fp16's largest value
+[[maybe_unused]] constexpr uint32_t kNotFinite = 0x80000000u;  // exponent of a token holding inf or NaN
+
+struct PairArgs {
+  float* y;
+  const uint8_t* wh;   // fp16 [N][K]
+  const uint8_t* wl;   // fp16 [N][K] or unused
+  const uint8_t* xh;   // fp16 [M][Kp] hi parts, then a plane of M rows of lo parts
+  const float* bias;
+  const int* xexp;     // [M]: row m of xh holds X row m times 2^-xexp[m]
+  const uint32_t* big; // non-zero: some scale of `col` is past kBigScale (or NULL)
+  const uint8_t* col;  // the column-major blocks wh and wl came from
+  size_t col_blocks;   // whole blocks in that buffer
+  const float* x;      // X as it came
+  float* part;         // [splits][M][N] partial planes (splits > 1)
+  uint32_t w_bytes;    // bytes of wh (and of wl)
+  uint32_t x_bytes;    // bytes of one xh plane (rows past M read zeros)
+  uint32_t y_bytes;    // M x N x 4
+  int M, N, K;
+  int steps;           // 64-K stages of a row (the last may be half)
+  int tiles_m, tiles_n;
+  int splits;
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t prsrc(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
+                                           0x00020000);
+}
+
+template <int MT, bool kWl>
+__global__ void __launch_bounds__(kPThreads, 1) gemm_pair_kernel(const PairArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (the buffer builtins exist only in the device pass)
+  constexpr int BM = 32 * MT;
+  constexpr int kTile = 2 * BM * kPRowBytes;
+  constexpr int kDx = 2 * BM / 64;          // X DMAs per wave and stage
+  constexpr int kWLoads = kWl ? 8 : 4;      // W loads per wave and stage
+  extern __shared__ __align__(16) uint8_t smem[];
+  const int t = threadIdx.x;
+  const int lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int lr = lane & 31;
+  const int h = lane >> 5;
+  const int m0 = (blockIdx.x % a.tiles_m) * BM;
+  const int n0 = (blockIdx.x / a.tiles_m) * kPBN;
+  const int z = blockIdx.y;
+  const int s0 = (int)((long long)a.steps * z / a.splits);
+  const int s1 = (int)((long long)a.steps * (z + 1) / a.splits);
+  const int steps = s1 - s0;
+
+  // X DMA: instruction i of wave w fills LDS rows 8 (8 i + w) .. + 7 of the
+  // slot (rows BM .. 2 BM - 1 are the lo parts).
+  const uint32_t x_row = (uint32_t)a.steps * kPRowBytes;
+  const __amdgpu_buffer_rsrc_t xrs = prsrc(a.xh, a.x_bytes);
+  const __amdgpu_buffer_rsrc_t xls = prsrc(a.xh + a.x_bytes, a.x_bytes);
+  uint32_t xvoff[kDx];
+#pragma unroll
+  for (int i = 0; i < kDx; i++) {
+    const int row = 8 * (8 * i + wave) + (lane >> 3);
+    const int c = (lane & 7) ^ ((row >> 1) & 7);
+    xvoff[i] = (uint32_t)(m0 + row % BM) * x_row + (uint32_t)c * 16u;
+  }
+  auto issue_x = [&](int s) __attribute__((always_inline)) {  // stage min(s, steps-1) -> slot of s
+    const int soff = (s0 + (s < steps ? s : steps - 1)) * kPRowBytes;
+    uint8_t* slot = smem + (s % kPRing) * kTile;
+#pragma unroll
+    for (int i = 0; i < kDx; i++) {
+      const bool lo = 8 * (8 * i + wave) >= BM;  // wave-uniform
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          lo ? xls : xrs,
+          (__attribute__((address_space(3))) void*)(slot + 8 * (8 * i + wave) * kPRowBytes), 16,
+          xvoff[i], soff, 0, 0);
+    }
+  };
+
+  // W: lane (n, h) holds elements 32 h .. + 31 of column n's stage; MFMA j
+  // takes 8 j .. + 7 of them.  Columns past N re-read column N - 1; elements
+  // past K read as zeros (their own row's end is not the buffer's).
+  const int ncol = n0 + 32 * wave + lr;
+  const bool nvalid = ncol < a.N;
+  const __amdgpu_buffer_rsrc_t whs = prsrc(a.wh, a.w_bytes);
+  const __amdgpu_buffer_rsrc_t wls = prsrc(kWl ? a.wl : a.wh, a.w_bytes);
+  const uint32_t wvoff = (uint32_t)min(ncol, a.N - 1) * (uint32_t)a.K * 2u + 64u * h;
+  struct Wreg {
+    u32x4 h[4], l[4];
+  };
+  auto load_w = [&](int s) __attribute__((always_inline)) -> Wreg {
+    const int sc = s0 + (s < steps ? s : steps - 1);
+    const uint32_t v = sc * kPStageK + 32 * h < a.K ? wvoff : 0xFFFFFF00u;
+    const uint32_t off = v == 0xFFFFFF00u ? v : v + (uint32_t)sc * kPRowBytes;
+    Wreg r;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      r.h[j] = __builtin_amdgcn_raw_buffer_load_b128(whs, off + 16 * j, 0, 0);
+      if constexpr (kWl) r.l[j] = __builtin_amdgcn_raw_buffer_load_b128(wls, off + 16 * j, 0, 0);
+    }
+    return r;
+  };
+
+  uint32_t aoff[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+    aoff[j] = (uint32_t)lr * kPRowBytes + (((4 * h + j) ^ ((lr >> 1) & 7)) << 4);
+  auto read_a = [&](int s, int i, int p, int j) __attribute__((always_inline)) -> half8 {
+    return *reinterpret_cast<const half8*>(smem + (s % kPRing) * kTile + aoff[j] +
+                                           (32 * i + BM * p) * kPRowBytes);
+  };
+
+  floatx16 acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[i][r] = 0.0f;
+
+  // Prologue: X of stages 0..2 in flight, stages 0 and 1 landed and published.
+  Wreg wa = load_w(0), wb;
+  asm volatile("" ::: "memory");
+  for (int i = 0; i < kPRing - 1; i++) issue_x(i);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kDx) : "memory");
+  half8 fa[2][4];  // hi and lo operands of the next row tile
+#pragma unroll
+  for (int p = 0; p < 2; p++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) fa[p][j] = read_a(0, 0, p, j);
+
+  floatx16 prev;  // the previous tile's stage sum
+#pragma unroll
+  for (int r = 0; r < 16; r++) prev[r] = 0.0f;
+
+  // At the end of stage s X(s+2), which went out in the stage before, has
+  // landed: this stage's X DMAs and W loads are all younger.
+  auto stage = [&](int s, const Wreg& w, Wreg& wn) __attribute__((always_inline)) {
+    issue_x(s + kPRing - 1);
+    asm volatile("" ::: "memory");
+    wn = load_w(s + 1);
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      const int ns = i + 1 == MT ? s + 1 : s, ni = (i + 1) % MT;
+      // The stage's products add up from zero and then to the tile's sum, so
+      // that sum is rounded once per 64 columns.
+      floatx16 p;
+#pragma unroll
+      for (int r = 0; r < 16; r++) p[r] = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const half8 bh = __builtin_bit_cast(half8, w.h[j]);
+        if constexpr (kWl)
+          p = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[0][j], __builtin_bit_cast(half8, w.l[j]),
+                                                     p, 0, 0, 0);
+        p = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[1][j], bh, p, 0, 0, 0);
+        fa[1][j] = read_a(ns, ni, 1, j);
+        p = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[0][j], bh, p, 0, 0, 0);
+        fa[0][j] = read_a(ns, ni, 0, j);
+      }
+      const int pi = (i + MT - 1) % MT;
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[pi][r] += prev[r];
+      prev = p;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kDx + kWLoads) : "memory");
+  };
+  int s = 0;
+  for (; s + 1 < steps; s += 2) {
+    stage(s, wa, wb);
+    stage(s + 1, wb, wa);
+  }
+  if (s < steps) stage(s, wa, wb);
+#pragma unroll
+  for (int r = 0; r < 16; r++) acc[MT - 1][r] += prev[r];
+  // Every DMA into LDS (the trailing re-reads included) has landed before
+  // the work-group's LDS is released.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+  // Register r of a lane holds output row m0 + 32 i + 8 (r / 4) + 4 h + r % 4,
+  // column ncol: scaled back by 2^xexp[m] (exact).  Y goes out through a
+  // buffer whose range is M x N, so rows past M drop out of range and lanes
+  // past N aim past it.  K pieces write their partial plane instead; the
+  // reduction adds the bias.
+  const __amdgpu_buffer_rsrc_t ers = prsrc(a.xexp, (uint32_t)a.M * 4u);
+  float* dst = a.splits > 1 ? a.part + (size_t)z * a.M * a.N : a.y;
+  const __amdgpu_buffer_rsrc_t yrs = prsrc(dst, a.y_bytes);
+  const float bv = (nvalid && a.bias && a.splits == 1) ? a.bias[ncol] : 0.0f;
+  // An output straight from the blocks, in fp32 over this piece: where a
+  // product n d leaves fp16 (a.big) or a token holds inf or NaN (its exponent
+  // says so), whose products with a zero wl would all be NaN.
+  auto from_blocks = [&](int m) -> float {
+    float v = 0.0f;
+    const int k1 = min(a.K, s1 * kPStageK);
+    for (int k = s0 * kPStageK; k < k1; k++) {
+      const size_t g = (size_t)k * (a.N / kBlockElems) + ncol / kBlockElems;
+      if (g >= a.col_blocks) continue;
+      const uint8_t* b = a.col + g * kBlockBytes;
+      const float d = f16_bits_to_f32((uint32_t)b[0] | ((uint32_t)b[1] << 8));
+      const int o = ncol % kBlockElems;
+      const int q = (b[2 + o / 2] >> (4 * (o & 1))) & 15;
+      v = fmaf((float)(q - 8), d * a.x[(size_t)m * a.K + k], v);
+    }
+    return v;
+  };
+  const bool big = kWl && *a.big != 0;
+#pragma unroll
+  for (int i = 0; i < MT; i++) {
+    uint32_t ex[16];
+    bool odd_row = big;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      ex[r] = __builtin_amdgcn_raw_buffer_load_b32(
+          ers, (uint32_t)(m0 + 32 * i + 8 * (r / 4) + 4 * h + r % 4) * 4u, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const uint32_t m = (uint32_t)(m0 + 32 * i + 8 * (r / 4) + 4 * h + r % 4);
+      const uint32_t off = nvalid ? (m * (uint32_t)a.N + (uint32_t)ncol) * 4u : 0xFFFFFFF0u;
+      if (kWl) odd_row = odd_row || ex[r] == kNotFinite;
+      const float v = ldexpf(acc[i][r], (int)ex[r]) + bv;
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), yrs, off, 0, 0);
+    }
+    if (kWl && odd_row && nvalid) {
+      for (int r = 0; r < 16; r++) {
+        const int m = m0 + 32 * i + 8 * (r / 4) + 4 * h + r % 4;
+        if (m < a.M && (big || (uint32_t)a.xexp[m] == kNotFinite))
+          dst[(size_t)m * a.N + ncol] = from_blocks(m) + bv;
+      }
+    }
+  }
+#endif
+}
+
+// W_col [m][nb blocks] -> wh, wl fp16 [32 nb][m].  A work-group of 256 threads
+// takes 64 inputs k by 8 block columns (256 outputs); thread (p, c) the blocks
+// (2 p, c) and (2 p + 1, c), so it holds pairs of neighbouring k for its 32
+// outputs and writes them as dwords into LDS rows of 33 (conflict-free: a
+// wave's lanes are 32 p at two c, 32 rows of 33 apart); the rows then leave as
+// whole 128-byte lines.  A scale past kBigScale sets *big (cleared by the
+// launch before): the GEMM then takes the blocks themselves.  Inputs past m and block columns past nb are skipped,
+// blocks past a short buffer are zero.
+constexpr int kExK = 64, kExC = 8;
+[[maybe_unused]] constexpr int kExPitch = 33;
+
+__global__ void __launch_bounds__(256)
+q4_0_col_expand_kernel(uint32_t* __restrict__ wh, uint32_t* __restrict__ wl,
+                       uint32_t* __restrict__ big, const uint8_t* __restrict__ w,
+                       uint32_t w_range, size_t avail, int nb, int m) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (the buffer builtins exist only in the device pass)
+  __shared__ uint32_t rows[kExC * 32 * kExPitch];
+  const int t = threadIdx.x;
+  const int p = t & 31, c = t >> 5;
+  const int k0 = blockIdx.y * kExK, c0 = blockIdx.x * kExC;
+  const __amdgpu_buffer_rsrc_t rs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w), (short)0, (int)w_range, 0x00020000);
+  uint32_t q[2][4], d[2];
+#pragma unroll
+  for (int e = 0; e < 2; e++) {
+    const int k = k0 + 2 * p + e;
+    const size_t g = (size_t)k * nb + c0 + c;
+    const bool ok = k < m && c0 + c < nb && g < avail;
+    const uint32_t byte = (uint32_t)(g * kBlockBytes);
+    const uint32_t off = ok ? byte & ~3u : 0xFFFFFF00u;
+    const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
+    const uint32_t b = __builtin_amdgcn_raw_buffer_load_b32(rs, off + 16, 0, 0);
+    const bool odd = (byte & 2) != 0;
+    const uint32_t sel = odd ? 0x07060504u : 0x05040302u;
+    const uint32_t v[5] = {a[0], a[1], a[2], a[3], b};
+#pragma unroll
+    for (int j = 0; j < 4; j++) q[e][j] = __builtin_amdgcn_perm(v[j + 1], v[j], sel);
+    d[e] = ok ? (odd ? v[0] >> 16 : v[0] & 0xFFFFu) : 0u;
+  }
+  if (max(d[0] & 0x7FFFu, d[1] & 0x7FFFu) > kBigScale) *big = 1;
+  uint32_t lo[32];
+  uint32_t* row = rows + (c * 32) * kExPitch + p;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const u32x4 n0 = unpack8(q[0][j]), n1 = unpack8(q[1][j]);
+    const half2v d0 = __builtin_bit_cast(half2v, d[0] | (d[0] << 16));
+    const half2v d1 = __builtin_bit_cast(half2v, d[1] | (d[1] << 16));
+#pragma unroll
+    for (int i = 0; i < 4; i++) {  // slots i: elements i and i + 4
+      const uint32_t u0 = n0[i], u1 = n1[i];
+      const half2v a0 = __builtin_bit_cast(half2v, u0), a1 = __builtin_bit_cast(half2v, u1);
+      const half2v h0 = a0 * d0, h1 = a1 * d1;
+      const half2v l0 = __builtin_elementwise_fma(a0, d0, -h0);
+      const half2v l1 = __builtin_elementwise_fma(a1, d1, -h1);
+      const half2v hp[2] = {{h0[0], h1[0]}, {h0[1], h1[1]}};
+      const half2v lp[2] = {{l0[0], l1[0]}, {l0[1], l1[1]}};
+#pragma unroll
+      for (int x = 0; x < 2; x++) {
+        const int o = 8 * j + i + 4 * x;
+        row[o * kExPitch] = __builtin_bit_cast(uint32_t, hp[x]);
+        lo[o] = __builtin_bit_cast(uint32_t, lp[x]);
+      }
+    }
+  }
+  // 256 output rows of 32 dwords (pairs of k): 8 lanes a row, 4 dwords each.
+  const size_t pitch = (size_t)m / 2;  // m is even
+  auto put = [&](uint32_t* out) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int r = i * 32 + (t >> 3), dw = (t & 7) * 4;
+      const int j = c0 * 32 + r;
+      if (j < nb * 32 && k0 / 2 + dw < (int)pitch) {
+        const uint32_t* s = rows + r * kExPitch + dw;
+        u32x4 v = {s[0], s[1], s[2], s[3]};
+        *reinterpret_cast<u32x4*>(out + (size_t)j * pitch + k0 / 2 + dw) = v;
+      }
+    }
+  };
+  __syncthreads();
+  put(wh);
+  __syncthreads();
+#pragma unroll
+  for (int o = 0; o < 32; o++) row[o * kExPitch] = lo[o];
+  __syncthreads();
+  put(wl);
+#endif
+}
+
+size_t rup(size_t v, size_t a) { return (v + a - 1) / a * a; }
+
+size_t pair_x_bytes(size_t batch, size_t m) {
+  return rup(2 * batch * rup(m, kPStageK) * 2, 256) + rup(batch * 4, 256);
+}
+
+// Rows per tile and K pieces.  Costs (microseconds): a 64-K stage 0.8 / 1.0 /
+// 1.5 on 32- / 64- / 128-row tiles, a round of work-groups ~3 more, the
+// reduction of K pieces its launch (~2.5) and a read of the planes (~4 TB/s).
+struct PairPlan {
+  int mt, splits;
+};
+PairPlan pair_plan(size_t n, size_t m, size_t batch, int num_cus) {
+  const size_t tn = (n + kPBN - 1) / kPBN;
+  const size_t steps = rup(m, kPStageK) / kPStageK;
+  PairPlan best{1, 1};
+  double best_cost = 1e300;
+  for (int mt : {1, 2, 4}) {
+    if (mt > 1 && (size_t)16 * mt >= batch) break;  // taller tiles than the rows
+    const size_t tiles = (batch + 32 * mt - 1) / (32 * mt) * tn;
+    const double stage_us = mt == 4 ? 1.5 : mt == 2 ? 1.0 : 0.8;
+    for (size_t sp = 1; sp <= std::min<size_t>(steps, 64); sp++) {
+      const size_t rounds = (tiles * sp + num_cus - 1) / num_cus;
+      double cost = (double)rounds * ((double)((steps + sp - 1) / sp) * stage_us + 3.0);
+      if (sp > 1) cost += 2.5 + (double)sp * (double)(batch * n * 4) / 4.0e6;
+      if (cost < best_cost * 0.999) {
+        best_cost = cost;
+        best = PairPlan{mt, (int)sp};
+      }
+      if (rounds > 1 && sp > 1) break;  // more pieces only add rounds
+    }
+  }
+  return best;
+}
+
+bool pair_shape_ok(size_t n, size_t m, size_t batch) {
+  const size_t lim = ((size_t)1 << 32) - 4096;
+  return n <= 0x7FFFFFF && m <= 0x7FFFFFF && batch <= 0x7FFFFFF && n * m * 2 < lim &&
+         (batch + 256) * rup(m, kPStageK) * 2 < lim && (batch + 256) * n * 4 < lim;
+}
+
+int* pair_exponents(uint8_t* xws, size_t batch, size_t m) {
+  return reinterpret_cast<int*>(xws + rup(2 * batch * rup(m, kPStageK) * 2, 256));
+}
+
+// (X is already converted at xws.)  wl NULL: wh alone.
+hipError_t launch_pair(float* y, const void* wh, const void* wl, const uint32_t* big,
+                       const uint8_t* col, size_t col_blocks, const float* x, const float* bias,
+                       size_t n, size_t m, size_t batch, uint8_t* xws, int num_cus,
+                       hipStream_t s) {
+  const PairPlan p = pair_plan(n, m, batch, num_cus);
+  const size_t kp = rup(m, kPStageK);
+  const int* xexp = pair_exponents(xws, batch, m);
+  hipError_t e;
+  PairArgs a;
+  a.big = big;
+  a.col = col;
+  a.col_blocks = col_blocks;
+  a.x = x;
+  a.y = y;
+  a.wh = static_cast<const uint8_t*>(wh);
+  a.wl = static_cast<const uint8_t*>(wl);
+  a.xh = xws;
+  a.bias = bias;
+  a.xexp = xexp;
+  a.part = reinterpret_cast<float*>(xws + pair_x_bytes(batch, m));
+  a.w_bytes = (uint32_t)(n * m * 2);
+  a.x_bytes = (uint32_t)(batch * kp * 2);
+  a.y_bytes = (uint32_t)(batch * n * 4);
+  a.M = (int)batch;
+  a.N = (int)n;
+  a.K = (int)m;
+  a.steps = (int)(kp / kPStageK);
+  a.tiles_m = (int)((batch + 32 * p.mt - 1) / (32 * p.mt));
+  a.tiles_n = (int)((n + kPBN - 1) / kPBN);
+  a.splits = p.splits;
+  auto go = [&](auto kernel) -> hipError_t {
+    const int lds = kPRing * 2 * 32 * p.mt * kPRowBytes;
+    hipError_t le = set_lds_limit(reinterpret_cast<const void*>(kernel), lds);
+    if (le != hipSuccess) return le;
+    hipLaunchKernelGGL(kernel, dim3(a.tiles_m * a.tiles_n, p.splits), dim3(kPThreads), lds, s, a);
+    return hipGetLastError();
+  };
+  if (wl)
+    e = p.mt == 4   ? go(gemm_pair_kernel<4, true>)
+        : p.mt == 2 ? go(gemm_pair_kernel<2, true>)
+                    : go(gemm_pair_kernel<1, true>);
+  else
+    e = p.mt == 4   ? go(gemm_pair_kernel<4, false>)
+        : p.mt == 2 ? go(gemm_pair_kernel<2, false>)
+                    : go(gemm_pair_kernel<1, false>);
+  if (e != hipSuccess || p.splits == 1) return e;
+  return launch_split_reduce(y, a.part, bias, batch * n, n, p.splits, s);
+}
+
+size_t pair_bytes(size_t n, size_t m, size_t batch, int num_cus) {
+  const PairPlan p = pair_plan(n, m, batch, num_cus);
+  return pair_x_bytes(batch, m) + (p.splits > 1 ? (size_t)p.splits * batch * n * 4 : 0);
+}
+
+}  // namespace
+
+// Whole block columns and 64-K stages, windows as the one-token kernel reads
+// them (dword-aligned, the last block's 2 bytes of over-read inside the
+// buffer), 32-bit offsets.
+bool q4_0_col_gemm_ok(const uint8_t* w, size_t w_len, size_t n, size_t m, size_t batch) {
+  if (n == 0 || m == 0 || n % kBlockElems != 0 || m % kBlockElems != 0 || batch == 0) return false;
+  if (((uintptr_t)w & 3) != 0 || w_len >= 0xFFFFFF00u || !pair_shape_ok(n, m, batch)) return false;
+  const size_t avail = w_len / kBlockBytes;
+  return avail > 0 && (avail % 2 == 0 || w_len >= avail * kBlockBytes + 2);
+}
+
+size_t q4_0_col_gemm_workspace_bytes(size_t n, size_t m, size_t batch, int num_cus) {
+  return 256 + 2 * rup(n * m * 2, 256) + pair_bytes(n, m, batch, num_cus);
+}
+
+hipError_t launch_q4_0_col_gemm(float* y, const uint8_t* w, size_t w_len, const float* x,
+                                const float* bias, size_t n, size_t m, size_t batch, void* ws,
+                                int num_cus, hipStream_t s) {
+  uint32_t* big = static_cast<uint32_t*>(ws);
+  uint8_t* base = static_cast<uint8_t*>(ws) + 256;
+  const size_t plane = rup(n * m * 2, 256);
+  uint8_t* xws = base + 2 * plane;
+  const int nb = (int)(n / kBlockElems);
+  hipError_t e = launch_x_hilo(xws, pair_exponents(xws, batch, m), x, batch, m,
+                               rup(m, kPStageK), big, s);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(q4_0_col_expand_kernel,
+                     dim3((unsigned)((nb + kExC - 1) / kExC), (unsigned)((m + kExK - 1) / kExK)),
+                     dim3(256), 0, s, reinterpret_cast<uint32_t*>(base),
+                     reinterpret_cast<uint32_t*>(base + plane), big, w, (uint32_t)w_len,
+                     w_len / kBlockBytes, nb, (int)m);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  return launch_pair(y, base, base + plane, big, w, w_len / kBlockBytes, x, bias, n, m, batch, xws,
+                     num_cus, s);
+}
+
+// fp16 weights [n][m] as they are: K % 32 == 0, w 16-byte aligned.
+bool f16_pair_gemm_ok(const uint8_t* w, size_t n, size_t m, size_t batch) {
+  return n != 0 && m != 0 && m % 32 == 0 && batch != 0 && ((uintptr_t)w & 15) == 0 &&
+         pair_shape_ok(n, m, batch);
+}
+
+size_t f16_pair_gemm_workspace_bytes(size_t n, size_t m, size_t batch, int num_cus) {
+  return pair_bytes(n, m, batch, num_cus);
+}
+
+hipError_t launch_f16_pair_gemm(float* y, const uint8_t* w, const float* x, const float* bias,
+                                size_t n, size_t m, size_t batch, void* ws, int num_cus,
+                                hipStream_t s) {
+  uint8_t* xws = static_cast<uint8_t*>(ws);
+  hipError_t e = launch_x_hilo(xws, pair_exponents(xws, batch, m), x, batch, m,
+                               rup(m, kPStageK), nullptr, s);
+  if (e != hipSuccess) return e;
+  return launch_pair(y, w, nullptr, nullptr, nullptr, 0, x, bias, n, m, batch, xws, num_cus, s);
+}
+
+}  // namespace hypno

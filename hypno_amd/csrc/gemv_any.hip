@@ -41,8 +41,8 @@ struct AnyWin {
 template <int F, int L>
 __global__ void __launch_bounds__(kAThreads)
 gemv_any_kernel(float* __restrict__ y, const uint8_t* __restrict__ w, size_t w_bytes,
-                const float* __restrict__ x, const float* __restrict__ bias, int n, int B,
-                size_t y_tok) {
+                const uint16_t* __restrict__ tail, const float* __restrict__ x,
+                const float* __restrict__ bias, int n, int B, size_t y_tok) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (the buffer builtins exist only in the device pass)
   using FT = AnyFmt<F>;
   constexpr int kDw = FT::kDw, kDeep = FT::kDeep;
@@ -75,6 +75,9 @@ gemv_any_kernel(float* __restrict__ y, const uint8_t* __restrict__ w, size_t w_b
     off[r] = first + (uint32_t)k * (uint32_t)row_bytes + (uint32_t)l * FT::kBytes;
   }
   const int steps = (B + L - 1) / L;
+  // W ends 2 bytes into its last block's last window dword, which the buffer's
+  // whole dwords leave out: the lane of that block reads the 2 bytes.
+  const bool has_tail = tail && row0 + kGroups * kAR >= n;  // wave-uniform
   auto load = [&](int s, int r) __attribute__((always_inline)) -> AnyWin<F> {
     AnyWin<F> o;
     const uint32_t byte = off[r] + (uint32_t)s * (uint32_t)(L * FT::kBytes);
@@ -86,6 +89,7 @@ gemv_any_kernel(float* __restrict__ y, const uint8_t* __restrict__ w, size_t w_b
       for (int k = 0; k < 4; k++) o.v[4 * i + k] = q[k];
     }
     o.v[kDw - 1] = __builtin_amdgcn_raw_buffer_load_b32(rs, a + 4 * (kDw - 1), 0, 2);
+    if (has_tail && s * L + l == B - 1 && row0 + g * kAR + r == n - 1) o.v[kDw - 1] = *tail;
     return o;
   };
   AnyWin<F> win[kDeep][kAR];
@@ -194,8 +198,8 @@ bool gemv_any_ok(int fmt, const uint8_t* w, size_t w_len, size_t n, size_t m) {
 }
 
 template <int F>
-static hipError_t launch_any(float* y, const uint8_t* w, size_t w_bytes, const float* x,
-                             const float* bias, size_t rows, size_t n, size_t m, size_t batch,
+static hipError_t launch_any(float* y, const uint8_t* w, size_t w_bytes, const uint16_t* tail,
+                             const float* x, const float* bias, size_t n, size_t m, size_t batch,
                              hipStream_t s) {
   const int B = (int)(m / kBlockElems);
   const size_t lds = (size_t)B * 128;
@@ -205,8 +209,8 @@ static hipError_t launch_any(float* y, const uint8_t* w, size_t w_bytes, const f
     const size_t per = (size_t)kAWaves * (64 / L) * kAR;
     for (size_t t = 0; t < batch; t += 65535) {
       const unsigned cnt = (unsigned)(batch - t < 65535 ? batch - t : 65535);
-      hipLaunchKernelGGL(kernel, dim3((unsigned)((rows + per - 1) / per), cnt), dim3(kAThreads),
-                         lds, s, y + t * n, w, w_bytes, x + t * m, bias, (int)rows, B, n);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)((n + per - 1) / per), cnt), dim3(kAThreads), lds,
+                         s, y + t * n, w, w_bytes, tail, x + t * m, bias, (int)n, B, n);
       if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     return hipSuccess;
@@ -221,25 +225,14 @@ hipError_t launch_gemv_any(int fmt, float* y, const uint8_t* w, size_t w_len, co
                            const float* bias, size_t n, size_t m, size_t batch, hipStream_t s) {
   const size_t row_bytes =
       m / kBlockElems * (size_t)(fmt == kFmtQ8_0 ? kQ8BlockBytes : kBlockBytes);
-  // The last row's last window dword ends past W when N rows end at 2 mod 4;
-  // if the buffer ends there too, that row goes to the any-shape kernel.
-  size_t rows = n, w_bytes = (n * row_bytes + 3) / 4 * 4;
-  if (w_bytes > w_len) {
-    rows = n - 1;
-    w_bytes = rows * row_bytes;  // a multiple of 4: row_bytes is 2 mod 4, rows even
-  }
-  hipError_t e = hipSuccess;
-  if (rows)
-    e = fmt == kFmtQ8_0 ? launch_any<kFmtQ8_0>(y, w, w_bytes, x, bias, rows, n, m, batch, s)
-                        : launch_any<kFmtQ4_0>(y, w, w_bytes, x, bias, rows, n, m, batch, s);
-  for (size_t t = 0; rows < n && t < batch && e == hipSuccess; t++) {
-    const uint8_t* wr = w + rows * row_bytes;
-    const float* br = bias ? bias + rows : nullptr;
-    e = fmt == kFmtQ8_0
-            ? launch_q8_0_generic(y + t * n + rows, wr, x + t * m, br, 1, m, 1, s)
-            : launch_q4_0_generic(y + t * n + rows, wr, row_bytes, x + t * m, br, 1, m, 1, s);
-  }
-  return e;
+  // Whole dwords of W; where N rows end at 2 mod 4 and the buffer ends with
+  // them, the last 2 bytes go apart.
+  const size_t end = n * row_bytes;
+  const bool cut = (end & 3) != 0 && w_len < end + 2;
+  const size_t w_bytes = cut ? end - 2 : (end + 3) / 4 * 4;
+  const uint16_t* tail = cut ? reinterpret_cast<const uint16_t*>(w + end - 2) : nullptr;
+  return fmt == kFmtQ8_0 ? launch_any<kFmtQ8_0>(y, w, w_bytes, tail, x, bias, n, m, batch, s)
+                         : launch_any<kFmtQ4_0>(y, w, w_bytes, tail, x, bias, n, m, batch, s);
 }
 
 }  // namespace hypno

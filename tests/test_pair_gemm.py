@@ -1,0 +1,111 @@
+"""Batches on the fp16-pair GEMM: column-major Q4_0 at many tokens and fp16
+weights whose rows are no multiple of 64, at the edges of its tiles (row tiles
+of 32, 64 and 128 tokens, 256 output columns, 64-column stages cut in half),
+with short buffers, scales past fp16's products, infinities and biases."""
+import ctypes
+
+import numpy as np
+import pytest
+
+
+def _p(t):
+    return None if t is None else ctypes.c_void_p(t.data_ptr())
+
+
+def _col_f64(orc, wb, x, bias, n, m):
+    return np.stack([orc.matmul_q4_0_col_f64(wb, r, bias, n, m) for r in x])
+
+
+def _col(torch, wb, x, bias, n, m):
+    from hypno_amd import _lib
+    dw, dx = torch.from_numpy(wb).cuda(), torch.from_numpy(x).cuda()
+    db = torch.from_numpy(bias).cuda() if bias is not None else None
+    y = torch.full((x.shape[0], n), float("nan"), device="cuda")
+    st = _lib.load().hypno_hip_matmul_q4_0_col_dev(_p(y), _p(dw), wb.size, _p(dx), _p(db), n, m,
+                                                   x.shape[0], None)
+    assert st == 0
+    torch.cuda.synchronize()
+    return y.cpu().numpy()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,n,m,cut", [(40, 2080, 2080, 0), (33, 3104, 1056, 0),
+                                            (65, 1056, 1120, 0), (129, 1024, 1024, 18),
+                                            (128, 256, 2048, 0), (300, 544, 1056, 0),
+                                            (64, 1056, 1056, 18 * 33 * 100 + 7)])
+def test_col_major_many_tokens(orc, tokens, n, m, cut):
+    import torch
+    print(f"col tokens={tokens} n={n} m={m} cut={cut}", flush=True)
+    rng = np.random.default_rng(tokens + n)
+    wb = orc.quantize_q4_0((rng.standard_normal(n * m) * 0.02).astype(np.float32))
+    wb = np.ascontiguousarray(wb[:wb.size - cut])
+    x = rng.standard_normal((tokens, m)).astype(np.float32)
+    x[:, ::61] *= 20.0
+    bias = rng.standard_normal(n).astype(np.float32)
+    got = _col(torch, wb, x, bias, n, m)
+    ref = _col_f64(orc, wb, x, bias, n, m)
+    # fp32 sums and pairs exact to 2^-22: random error well under sqrt(K) 2^-22
+    for t in range(tokens):
+        assert orc.normwise_err(got[t], ref[t]) <= 2e-5, t
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [0x6FFF, 0x7000, 0x7BFF, 0x0001, 0x8200])
+def test_col_major_scale_range(orc, bits):
+    """One block's scale at the largest whose products fp16 holds, past it, at
+    fp16's largest value, at its smallest and at a negative subnormal."""
+    import torch
+    tokens, n, m = 40, 2080, 2080
+    rng = np.random.default_rng(bits)
+    wb = orc.quantize_q4_0((rng.standard_normal(n * m) * 0.02).astype(np.float32))
+    g = 777 * (n // 32) + 13
+    wb[18 * g:18 * g + 2] = np.frombuffer(np.uint16(bits).tobytes(), np.uint8)
+    x = rng.standard_normal((tokens, m)).astype(np.float32)
+    got = _col(torch, wb, x, None, n, m)
+    ref = _col_f64(orc, wb, x, None, n, m)
+    for t in range(tokens):
+        assert orc.normwise_err(got[t], ref[t]) <= 2e-5, t
+    # the other block columns on their own
+    keep = np.r_[0:13 * 32, 14 * 32:n]
+    for t in range(tokens):
+        assert orc.normwise_err(got[t][keep], ref[t][keep]) <= 2e-5, t
+
+
+@pytest.mark.gpu
+def test_col_major_infinite_token(orc):
+    import torch
+    tokens, n, m = 40, 2080, 2080
+    rng = np.random.default_rng(3)
+    wb = orc.quantize_q4_0((rng.standard_normal(n * m) * 0.02).astype(np.float32))
+    x = rng.standard_normal((tokens, m)).astype(np.float32)
+    x[7, 100] = np.inf
+    got = _col(torch, wb, x, None, n, m)
+    w = orc.dequantize_q4_0(wb).reshape(m, n)[100]
+    want = np.full(n, np.nan)
+    want[w != 0] = np.sign(w[w != 0]) * np.inf
+    assert np.array_equal(got[7], want.astype(np.float32), equal_nan=True)
+    ref = _col_f64(orc, wb, x[8:], None, n, m)
+    for t in range(8, tokens):
+        assert orc.normwise_err(got[t], ref[t - 8]) <= 2e-5, t
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,n,m", [(2, 20001, 1056), (16, 2600, 992), (33, 1300, 1120),
+                                        (65, 257, 2400), (129, 511, 1056), (300, 300, 544)])
+def test_f16_half_stage_rows(orc, tokens, n, m):
+    import torch
+
+    import hypno_amd as hk
+    print(f"f16 tokens={tokens} n={n} m={m}", flush=True)
+    rng = np.random.default_rng(tokens + n)
+    w = (rng.standard_normal(n * m) * 0.02).astype(np.float16)
+    x = rng.standard_normal((tokens, m)).astype(np.float32)
+    dw = torch.from_numpy(w.view(np.uint8)).cuda()
+    dx = torch.from_numpy(x).cuda()
+    y = torch.full((tokens, n), float("nan"), device="cuda")
+    hk.batch_matmul(y, dw, hk.DType.FP16, dx, n, m, tokens)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    ref = x.astype(np.float64) @ w.reshape(n, m).astype(np.float64).T
+    for t in range(tokens):
+        assert orc.normwise_err(got[t], ref[t]) <= 2e-5, t
