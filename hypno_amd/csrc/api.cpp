@@ -363,8 +363,8 @@ int q4_0_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const flo
 
 // Q8_0 (ops.rs:33-36, turbo.rs:334-341): the reference dequantises the
 // whole tensor and slices rows of it, so a buffer shorter than n*m elements
-// is a panic there (EINVAL here).  From 16 tokens the fp16 GEMM path runs
-// (weights expanded to fp16 once per call); 2 to 15 go through the few-row
+// is a panic there (EINVAL here).  From 16 tokens the MFMA GEMMs of
+// gemm_q8_0.hip run on activations rounded to fp16; 2 to 15 go through the few-row
 // GEMV in launches of 2 to 8 rows (the tokens split evenly), one token
 // through the GEMV.
 int q8_0_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const float* bias,
@@ -390,7 +390,7 @@ int q8_0_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const flo
   hipError_t e;
   if (batch >= kGemmMinBatch && q8_0_gemm_ok(n, m, batch)) {
     WsLock ws;
-    st = lock_workspace(ds, s, q8_0_gemm_workspace_bytes(batch, n, m, cus), ws,
+    st = lock_workspace(ds, s, q8_0_gemm_workspace_bytes(w, batch, n, m, cus), ws,
                         "Q8_0 GEMM workspace");
     if (st) return st;
     e = launch_q8_0_gemm(y, w, x, bias, n, m, batch, ws.p, cus, s);

@@ -244,9 +244,9 @@ hipError_t launch_quantize_q8_0(uint8_t* out, const float* src, size_t n_blocks,
 hipError_t launch_dequantize_q8_0(float* out, const uint8_t* q, size_t n_blocks, hipStream_t s);
 hipError_t launch_q8_0_generic(float* y, const uint8_t* w, const float* x, const float* bias,
                                size_t n, size_t m, size_t batch, hipStream_t s);
-// Q8_0 prefill through fp16 weights and the fp16 GEMM (gemm_q8_0.hip).
+// Q8_0 prefill: the block GEMM, or fp16 weights and the fp16 GEMM (gemm_q8_0.hip).
 bool q8_0_gemm_ok(size_t n, size_t m, size_t batch);
-size_t q8_0_gemm_workspace_bytes(size_t batch, size_t n, size_t m, int num_cus);
+size_t q8_0_gemm_workspace_bytes(const uint8_t* w, size_t batch, size_t n, size_t m, int num_cus);
 hipError_t launch_q8_0_gemm(float* y, const uint8_t* w, const float* x, const float* bias,
                             size_t n, size_t m, size_t batch, void* ws, int num_cus,
                             hipStream_t s);
@@ -388,6 +388,7 @@ hipError_t launch_q4_0_skinny(float* y, const uint8_t* w, const float* x, const 
 struct BlockPlan {
   int mt;      // 32-row tiles per wave
   int splits;  // K pieces
+  double cost; // of the kernel and its reduction, microseconds by the model
 };
 bool block_gemm_ok(int fmt, const uint8_t* w, size_t w_len, size_t n, size_t m, size_t batch);
 BlockPlan block_plan(size_t n, size_t m, size_t batch, int num_cus);
@@ -395,6 +396,15 @@ size_t block_gemm_workspace_bytes(const BlockPlan& p, size_t n, size_t m, size_t
 hipError_t launch_block_gemm(const BlockPlan& p, int fmt, float* y, const uint8_t* w,
                              const float* x, const float* bias, size_t n, size_t m, size_t batch,
                              void* ws, hipStream_t s);
+
+// The same kernel on x rounded once to fp16 (xh [rows][m], x_bytes of it, and
+// its exponents), m % 64 == 0, rows permuted for Q4_0 as launch_x_f16_permuted
+// writes them; `part` holds p.splits planes.
+BlockPlan block_plan_f16x(int fmt, size_t n, size_t m, size_t batch, int num_cus, size_t planes);
+hipError_t launch_block_gemm_f16x(const BlockPlan& p, int fmt, float* y, const uint8_t* w,
+                                  const float* bias, size_t n, size_t m, size_t batch,
+                                  const void* xh, size_t x_bytes, const int* xexp, float* part,
+                                  hipStream_t s);
 
 // X fp32 [batch][m] -> fp16 [batch][kp] hi parts and a plane of lo parts in
 // natural column order, per-row exponents at xexp; with `clear`, *clear = 0
@@ -432,6 +442,9 @@ hipError_t launch_x_rows_f16(const float* x, size_t batch, size_t rows, size_t m
 // X -> fp16 [Mp][K] in natural column order, rows scaled as above
 // (FP16-weight GEMM pre-pass).
 hipError_t launch_x_f16_plain(const float* x, size_t batch, size_t m, void* ws, hipStream_t s);
+// Either of the two in one read of x where its rows allow it (gemm_exact.hip).
+hipError_t launch_x_f16_onepass(const float* x, size_t batch, size_t m, void* ws, bool permute,
+                                hipStream_t s);
 // DMA-fed FP16-weight GEMM (gemm_q4.hip).
 bool f16_gemm_v2_ok(const uint8_t* w, size_t n, size_t m, size_t batch);
 size_t f16_gemm_v2_workspace_bytes(size_t batch, size_t n, size_t m, int num_cus);

@@ -31,6 +31,13 @@
 //    issues its MFMAs, the reloads of the A registers they free for slot
 //    j + 2, the 16 scale FMAs of slot j - 1 and a share of the next block's
 //    unpack, in that order (a scheduling barrier between slots).
+//  * One part: x rounded once to fp16 (the prefill GEMMs' arithmetic) takes
+//    the same kernel without the lo rows, half the MFMAs and half the LDS per
+//    row, so tiles go up to 256 rows.  Per 256 x 256 x 64 stage 2.3 us with
+//    every CU at work (930 TFLOP/s); copies without X and W DMA 13% faster,
+//    without the barrier 4%, without the A reads no faster: what is left is
+//    the MFMAs and FMAs of two waves on one issue port (a probe of 32x32x16
+//    MFMAs with 8 FMAs each reaches 1560 TFLOP/s, with 10 ops 1460).
 //  * K % 64 == 32: the X rows are padded with a zero block, and the scale of
 //    the block past the row's end is taken as 0.  Rows of an odd number of
 //    blocks start on 2-byte boundaries: each row's window then starts at the
@@ -54,13 +61,13 @@ constexpr int kBRowBytes = kBStageK * 2;
 
 // FMT: weight format; MT: 32-row tiles per wave; ODD: an odd number of blocks
 // per row.
-template <int FMT, int MT, bool ODD>
+template <int FMT, int MT, bool ODD, int PARTS = 2>
 struct BlockGeom {
   static constexpr int kBlk = FMT == kFmtQ8_0 ? kQ8BlockBytes : kBlockBytes;
   static constexpr int kRowDw = 2 * kBlk / 4 + (ODD ? 1 : 0);  // a row's dwords per stage
   static constexpr int kDw = (32 * kRowDw + 63) / 64;          // W DMAs per wave and stage
   static constexpr int kWSlot = 256 * kDw;
-  static constexpr int kXRows = 64 * MT;  // hi rows, then lo rows
+  static constexpr int kXRows = 32 * PARTS * MT;  // hi rows, then lo rows
   static constexpr int kTile = kXRows * kBRowBytes;
   static constexpr int kDx = kXRows / 64;  // X DMAs per wave and stage
   static_assert(kXRows % 64 == 0, "every wave issues the same number of X DMAs");
@@ -109,13 +116,13 @@ struct RawBlock {
   uint32_t d;
 };
 
-template <int FMT, int MT, bool ODD>
+template <int FMT, int MT, bool ODD, int PARTS>
 __global__ void __launch_bounds__(kBThreads, 1) gemm_block_kernel(const BlockArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)  // (the buffer builtins exist only in the device pass)
-  using G = BlockGeom<FMT, MT, ODD>;
+  using G = BlockGeom<FMT, MT, ODD, PARTS>;
   constexpr int BM = 32 * MT;
   constexpr int kRing = G::kRing, kWRing = G::kWRing;
-  constexpr int kParts = 2;  // hi, lo
+  constexpr int kParts = PARTS;  // hi, lo; or the rounded x alone
   extern __shared__ __align__(16) uint8_t smem[];
   const int t = threadIdx.x;
   const int lane = t & 63;
@@ -158,7 +165,7 @@ __global__ void __launch_bounds__(kBThreads, 1) gemm_block_kernel(const BlockArg
     uint8_t* slot = smem + (s % kRing) * G::kTile;
 #pragma unroll
     for (int i = 0; i < G::kDx; i++) {
-      const bool lo = 8 * (8 * i + wave) >= BM;  // wave-uniform
+      const bool lo = PARTS == 2 && 8 * (8 * i + wave) >= BM;  // wave-uniform
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           lo ? xls : xrs,
           (__attribute__((address_space(3))) void*)(slot + 8 * (8 * i + wave) * kBRowBytes), 16,
@@ -523,7 +530,7 @@ size_t rup(size_t v, size_t a) { return (v + a - 1) / a * a; }
 BlockPlan block_plan(size_t n, size_t m, size_t batch, int num_cus) {
   const size_t tn = (n + kBN - 1) / kBN;
   const size_t steps = rup(m, kBStageK) / kBStageK;
-  BlockPlan best{1, 1};
+  BlockPlan best{1, 1, 0.0};
   double best_cost = 1e300;
   for (int mt : {1, 2, 4}) {
     if (mt > 1 && (size_t)16 * mt >= batch) break;  // taller tiles than the rows
@@ -537,8 +544,35 @@ BlockPlan block_plan(size_t n, size_t m, size_t batch, int num_cus) {
       if (sp > 1) cost += 2.5 + (double)sp * (double)(batch * n * 4) / 4.0e6;
       if (cost < best_cost * 0.999) {
         best_cost = cost;
-        best = BlockPlan{mt, (int)sp};
+        best = BlockPlan{mt, (int)sp, cost};
       }
+      if (rounds > 1 && sp > 1) break;  // more pieces only add rounds
+    }
+  }
+  return best;
+}
+
+// The same for x rounded once to fp16 (m % 64 == 0), with no more than
+// `planes` bytes of partial planes.  A stage costs 0.95 / 1.25 / 2.3 on 64- /
+// 128- / 256-row tiles (Q8_0, twice the weight bytes: 1.0 / 1.42 / 2.35); K
+// pieces write planes that the reduction reads, ~3 TB/s in all.
+BlockPlan block_plan_f16x(int fmt, size_t n, size_t m, size_t batch, int num_cus, size_t planes) {
+  const size_t tn = (n + kBN - 1) / kBN;
+  const size_t steps = m / kBStageK;
+  BlockPlan best{2, 1, 1e300};
+  for (int mt : {2, 4, 8}) {
+    if (mt > 2 && (size_t)16 * mt >= batch) break;  // taller tiles than the rows
+    const size_t tm = (batch + 32 * mt - 1) / (32 * mt);
+    const size_t tiles = tm * tn;
+    const bool q8 = fmt == kFmtQ8_0;
+    const double stage_us = mt == 8 ? (q8 ? 2.35 : 2.3) : mt == 4 ? (q8 ? 1.42 : 1.25)
+                                                                  : (q8 ? 1.0 : 0.95);
+    for (size_t sp = 1; sp <= std::min<size_t>(steps, 64); sp++) {
+      if (sp > 1 && sp * batch * n * 4 > planes) break;
+      const size_t rounds = (tiles * sp + num_cus - 1) / num_cus;
+      double cost = (double)rounds * ((double)((steps + sp - 1) / sp) * stage_us + 3.0);
+      if (sp > 1) cost += 2.5 + (double)sp * (double)(batch * n * 4) / 3.0e6;
+      if (cost < best.cost * 0.999) best = BlockPlan{mt, (int)sp, cost};
       if (rounds > 1 && sp > 1) break;  // more pieces only add rounds
     }
   }
@@ -578,9 +612,9 @@ static hipError_t launch_block_mt(const BlockPlan& p, const BlockArgs& a, hipStr
     hipLaunchKernelGGL(kernel, dim3(a.tiles_m * a.tiles_n, p.splits), dim3(kBThreads), lds, s, a);
     return hipGetLastError();
   };
-  if (p.mt == 4) return go(gemm_block_kernel<FMT, 4, ODD>, BlockGeom<FMT, 4, ODD>::kLds);
-  if (p.mt == 2) return go(gemm_block_kernel<FMT, 2, ODD>, BlockGeom<FMT, 2, ODD>::kLds);
-  return go(gemm_block_kernel<FMT, 1, ODD>, BlockGeom<FMT, 1, ODD>::kLds);
+  if (p.mt == 4) return go(gemm_block_kernel<FMT, 4, ODD, 2>, BlockGeom<FMT, 4, ODD>::kLds);
+  if (p.mt == 2) return go(gemm_block_kernel<FMT, 2, ODD, 2>, BlockGeom<FMT, 2, ODD>::kLds);
+  return go(gemm_block_kernel<FMT, 1, ODD, 2>, BlockGeom<FMT, 1, ODD>::kLds);
 }
 
 hipError_t launch_block_gemm(const BlockPlan& p, int fmt, float* y, const uint8_t* w,
@@ -622,6 +656,47 @@ hipError_t launch_block_gemm(const BlockPlan& p, int fmt, float* y, const uint8_
     e = odd ? launch_block_mt<kFmtQ4_0, true>(p, a, s) : launch_block_mt<kFmtQ4_0, false>(p, a, s);
   if (e != hipSuccess || p.splits == 1) return e;
   return launch_split_reduce(y, a.part, bias, batch * n, n, p.splits, s);
+}
+
+template <int FMT>
+static hipError_t launch_block_single(const BlockPlan& p, const BlockArgs& a, hipStream_t s) {
+  auto go = [&](auto kernel, int lds) -> hipError_t {
+    hipError_t e = set_lds_limit(reinterpret_cast<const void*>(kernel), lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kernel, dim3(a.tiles_m * a.tiles_n, p.splits), dim3(kBThreads), lds, s, a);
+    return hipGetLastError();
+  };
+  if (p.mt == 8) return go(gemm_block_kernel<FMT, 8, false, 1>, BlockGeom<FMT, 8, false, 1>::kLds);
+  if (p.mt == 4) return go(gemm_block_kernel<FMT, 4, false, 1>, BlockGeom<FMT, 4, false, 1>::kLds);
+  return go(gemm_block_kernel<FMT, 2, false, 1>, BlockGeom<FMT, 2, false, 1>::kLds);
+}
+
+hipError_t launch_block_gemm_f16x(const BlockPlan& p, int fmt, float* y, const uint8_t* w,
+                                  const float* bias, size_t n, size_t m, size_t batch,
+                                  const void* xh, size_t x_bytes, const int* xexp, float* part,
+                                  hipStream_t s) {
+  BlockArgs a;
+  a.y = y;
+  a.w = w;
+  a.xh = static_cast<const uint8_t*>(xh);
+  a.bias = bias;
+  a.xexp = xexp;
+  a.part = part;
+  a.B = (int)(m / kBlockElems);
+  a.w_bytes = (uint32_t)(n * a.B * (fmt == kFmtQ8_0 ? kQ8BlockBytes : kBlockBytes));
+  a.x_bytes = (uint32_t)x_bytes;
+  a.y_bytes = (uint32_t)(batch * n * 4);
+  a.M = (int)batch;
+  a.N = (int)n;
+  a.steps = (int)(m / kBStageK);
+  a.tiles_m = (int)((batch + 32 * p.mt - 1) / (32 * p.mt));
+  a.tiles_n = (int)((n + kBN - 1) / kBN);
+  a.xcd_map = (a.tiles_m * a.tiles_n) % 8 == 0 ? 1 : 0;
+  a.splits = p.splits;
+  hipError_t e = fmt == kFmtQ8_0 ? launch_block_single<kFmtQ8_0>(p, a, s)
+                                 : launch_block_single<kFmtQ4_0>(p, a, s);
+  if (e != hipSuccess || p.splits == 1) return e;
+  return launch_split_reduce(y, part, bias, batch * n, n, p.splits, s);
 }
 
 hipError_t launch_split_reduce(float* y, const float* part, const float* bias, size_t mn, size_t n,

@@ -426,10 +426,11 @@ exact_split_reduce_kernel(float* __restrict__ y, const float* __restrict__ part,
 // 8 columns (group g = t + 256 u, u < kXGroups) in registers while the row's
 // largest |x| is found, then writes them scaled by 2^sh (sh puts that
 // maximum in [2^14, 2^15); 0 for an all-zero row or one holding inf or NaN,
-// the same rule as x_row_to_f16) and rounded to fp16, each group permuted to
-// the unpack order e0,e4,e1,e5,e2,e6,e3,e7; xexp[row] = -sh.  Rows M..Mp-1
+// the same rule as x_row_to_f16) and rounded to fp16, with kPerm each group
+// permuted to the unpack order e0,e4,e1,e5,e2,e6,e3,e7; xexp[row] = -sh.  Rows M..Mp-1
 // are written as zeros.  K <= 256 * 8 * kXGroups.
 constexpr int kXGroups = 8;
+template <bool kPerm>
 __global__ void __launch_bounds__(256)
 x_rows_f16_onepass_kernel(u32x4* __restrict__ xh, int* __restrict__ xexp,
                           const float* __restrict__ x, int M, int K) {
@@ -481,8 +482,9 @@ x_rows_f16_onepass_kernel(u32x4* __restrict__ xh, int* __restrict__ xexp,
       u32x4 packed;
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        const uint32_t lo = __builtin_bit_cast(uint16_t, (_Float16)ldexpf(e[perm[2 * j]], sh));
-        const uint32_t hi = __builtin_bit_cast(uint16_t, (_Float16)ldexpf(e[perm[2 * j + 1]], sh));
+        const int i0 = kPerm ? perm[2 * j] : 2 * j, i1 = kPerm ? perm[2 * j + 1] : 2 * j + 1;
+        const uint32_t lo = __builtin_bit_cast(uint16_t, (_Float16)ldexpf(e[i0], sh));
+        const uint32_t hi = __builtin_bit_cast(uint16_t, (_Float16)ldexpf(e[i1], sh));
         packed[j] = lo | (hi << 16);
       }
       dst[g] = packed;
@@ -493,11 +495,13 @@ x_rows_f16_onepass_kernel(u32x4* __restrict__ xh, int* __restrict__ xexp,
 
 size_t rup(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
-// Geometry chosen for a shape: M-tiles per wave and K pieces.
+// Geometry chosen for a shape: M-tiles per wave and K pieces, and what the
+// cost model below makes of it.
 struct ExactPlan {
   int mt;
   int tiles_m, tiles_n;
   int splits;
+  double cost;
 };
 
 // Tile height and K pieces by a cost model of this kernel on the MI355X
@@ -509,7 +513,7 @@ struct ExactPlan {
 ExactPlan exact_plan(size_t batch, size_t n, size_t m, int num_cus) {
   const size_t tn = (n + kEBN - 1) / kEBN;
   const size_t steps = m / kEStageK;
-  ExactPlan best{8, 1, (int)tn, 1};
+  ExactPlan best{8, 1, (int)tn, 1, 0.0};
   double best_cost = 1e300;
   for (int mt : {1, 2, 4, 8, 16}) {
     if (mt > 1 && (size_t)16 * (mt / 2) >= batch) break;  // taller tiles than the rows
@@ -523,13 +527,27 @@ ExactPlan exact_plan(size_t batch, size_t n, size_t m, int num_cus) {
       if (sp > 1) cost += 2.5 + (double)sp * (double)(batch * n * 4) / 4.0e6;
       if (cost < best_cost * 0.999) {
         best_cost = cost;
-        best = ExactPlan{mt, (int)tm, (int)tn, (int)sp};
+        best = ExactPlan{mt, (int)tm, (int)tn, (int)sp, cost};
       }
       if (rounds > 1 && sp > 1) break;  // more pieces only add rounds
     }
   }
   return best;
 }
+
+size_t planes_bytes(int splits, size_t batch, size_t n) {
+  return splits > 1 ? (size_t)splits * batch * n * 4 : 0;
+}
+
+// Whether the block GEMM on the same fp16 rows (32x32x16 MFMAs, 256 columns a
+// work-group) is the faster of the two: its 256 x 256 tiles spend half the
+// stages and LDS reads of this kernel's 256 x 128 ones per product, where a
+// grid of them comes out even.  The factor is what this kernel's tall tiles
+// measured above the model on a full chip (3 to 8%).  Per call, this kernel
+// and the other (us): 2048 x 14336, K 4096: 375 / 296; 1024 x 14336, K 4096:
+// 210 / 155; 2048 x 5632, K 2048: 96 / 83; left here: 512 x 8192, K 3072:
+// 53.5 / 55.0; 512 x 3072, K 8192: 54.2 / 55.7; 2048 x 2048, K 5632: 85 / 87.
+bool use_block(const ExactPlan& p, const BlockPlan& b) { return b.cost < 1.05 * p.cost; }
 
 }  // namespace
 
@@ -549,31 +567,45 @@ bool q4_0_gemm_exact_ok(const uint8_t* w, size_t w_len, size_t n, size_t m, size
 size_t q4_0_gemm_exact_workspace_bytes(size_t batch, size_t n, size_t m, int num_cus) {
   const ExactPlan p = exact_plan(batch, n, m, num_cus);
   const size_t xb = rup(gemm_workspace_bytes(batch, m), 256);
-  return p.splits > 1 ? xb + (size_t)p.splits * batch * n * 4 : xb;
+  return xb + planes_bytes(p.splits, batch, n);
+}
+
+hipError_t launch_x_f16_onepass(const float* x, size_t batch, size_t m, void* ws, bool permute,
+                                hipStream_t s) {
+  if (m > (size_t)256 * 8 * kXGroups || ((uintptr_t)x & 15) != 0)
+    return permute ? launch_x_f16_permuted(x, batch, m, ws, s)
+                   : launch_x_f16_plain(x, batch, m, ws, s);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)rup(batch, 128)), dim3(256), 0, s,
+                       static_cast<u32x4*>(ws), gemm_x_exponents(ws, batch, m), x, (int)batch,
+                       (int)m);
+    return hipGetLastError();
+  };
+  return permute ? go(x_rows_f16_onepass_kernel<true>) : go(x_rows_f16_onepass_kernel<false>);
 }
 
 hipError_t launch_q4_0_gemm_exact(float* y, const uint8_t* w, const float* x, const float* bias,
                                   size_t n, size_t m, size_t batch, void* ws, int num_cus,
                                   hipStream_t s) {
-  hipError_t e;
-  if (m <= (size_t)256 * 8 * kXGroups && ((uintptr_t)x & 15) == 0) {
-    hipLaunchKernelGGL(x_rows_f16_onepass_kernel, dim3((unsigned)rup(batch, 128)), dim3(256), 0, s,
-                       static_cast<u32x4*>(ws), gemm_x_exponents(ws, batch, m), x, (int)batch,
-                       (int)m);
-    e = hipGetLastError();
-  } else {
-    e = launch_x_f16_permuted(x, batch, m, ws, s);
-  }
+  hipError_t e = launch_x_f16_onepass(x, batch, m, ws, true, s);
   if (e != hipSuccess) return e;
   const ExactPlan p = exact_plan(batch, n, m, num_cus);
+  const size_t xb = rup(gemm_workspace_bytes(batch, m), 256);
+  // (the workspace is the other plan's: a block plan whose partial planes
+  // need more is not taken)
+  const BlockPlan b = block_plan_f16x(kFmtQ4_0, n, m, batch, num_cus,
+                                      planes_bytes(p.splits, batch, n));
+  if (use_block(p, b))
+    return launch_block_gemm_f16x(b, kFmtQ4_0, y, w, bias, n, m, batch, ws,
+                                  rup(batch, 128) * m * 2, gemm_x_exponents(ws, batch, m),
+                                  reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + xb), s);
   ExactArgs a;
   a.y = y;
   a.w = w;
   a.xh = static_cast<const uint8_t*>(ws);
   a.bias = bias;
   a.xexp = gemm_x_exponents(ws, batch, m);
-  a.part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) +
-                                    rup(gemm_workspace_bytes(batch, m), 256));
+  a.part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + xb);
   a.w_bytes = (uint32_t)(n * (m / kBlockElems) * kBlockBytes);
   a.x_bytes = (uint32_t)(rup(batch, 128) * m * 2);
   a.xe_bytes = (uint32_t)(rup(batch, 128) * 4);

@@ -1,9 +1,19 @@
 // Q8_0 prefill (turbo.rs:334-341 dequantises the tensor to fp32 and runs one
-// matmul_f32 per token).  Here, for M >= 16 tokens: the weights are expanded
-// once per call to fp16 in a workspace and an fp16 MFMA GEMM runs on them
+// matmul_f32 per token).  Here, for M >= 16 tokens with the activations
+// rounded to fp16 as on the other GEMM paths, one of two ways:
+//
+// The block GEMM (gemm_block.hip) reads the blocks themselves: exact integers
+// on the matrix cores, each block's scale in fp32.  No expansion pass (3 bytes
+// moved per weight: 40 us for 14336 x 4096, as long as the product at 128
+// tokens) and no rounding of the weights.  Per call, expanded and block (us):
+// 14336 x 4096: 62.6 / 28.8 at 16 tokens, 80.8 / 43.8 at 128, 126 / 111 at
+// 512, 353 / 325 at 2048; 4096 x 14336: 88 / 45 at 128, 141 / 108 at 512.
+//
+// Expanded once per call to fp16 in a workspace, then an fp16 MFMA GEMM
 // (gemm_q4.hip: the register-streaming kernel up to 64 tokens, the DMA-fed
-// one beyond), with the activations rounded to fp16 as on the other GEMM
-// paths.
+// one beyond), which spends no VALU on scales: long prompts on few rows (4096
+// x 14336, 2048 tokens: 322 against 362 us) and weights at odd 2-byte
+// addresses.
 //
 // Each row n is expanded as (u - 128) * (d / D_n), D_n = the row's largest
 // |d|: every value then lies in [-128, 128], so none overflows fp16 (a plain
@@ -85,7 +95,30 @@ bool q8_0_use_stream(size_t n, size_t m, size_t batch) {
   return batch <= 64 &&
          f16_gemm_stream_ok(reinterpret_cast<const uint8_t*>((uintptr_t)256), nullptr, n, m, batch);
 }
-size_t q8_0_gemm_workspace_bytes(size_t batch, size_t n, size_t m, int num_cus) {
+
+// The block GEMM's plan, or splits = 0 where the expanded weights are faster:
+// from one work-group of 128 x 256 per CU that way costs about 3 + 0.62 us per
+// million weights to expand and, a round, 3 + 1.1 us per 64 columns of K.  Up
+// to 64 MB of partial planes (the expansion needs more than that anyway).
+static BlockPlan q8_0_plan(const uint8_t* w, size_t n, size_t m, size_t batch, int num_cus) {
+  const size_t bytes = n * (m / kBlockElems) * kQ8BlockBytes;
+  if (!block_gemm_ok(kFmtQ8_0, w, bytes, n, m, batch)) return BlockPlan{0, 0, 0.0};
+  const BlockPlan b = block_plan_f16x(kFmtQ8_0, n, m, batch, num_cus, (size_t)64 << 20);
+  const size_t tiles = (n + 255) / 256 * ((batch + 127) / 128);
+  if (tiles >= (size_t)num_cus) {
+    const double rounds = (double)((tiles + num_cus - 1) / num_cus);
+    if (3.0 + 0.62e-6 * (double)n * m + rounds * (3.0 + 1.1 * (m / 64)) < b.cost)
+      return BlockPlan{0, 0, 0.0};
+  }
+  return b;
+}
+
+size_t q8_0_gemm_workspace_bytes(const uint8_t* w, size_t batch, size_t n, size_t m,
+                                 int num_cus) {
+  const BlockPlan b = q8_0_plan(w, n, m, batch, num_cus);
+  if (b.splits)
+    return round256(gemm_workspace_bytes(batch, m)) +
+           (b.splits > 1 ? (size_t)b.splits * batch * n * 4 : 0);
   return round256(n * m * 2) + round256(n * 4) +
          (q8_0_use_stream(n, m, batch) ? f16_gemm_stream_workspace_bytes(batch, n, m, num_cus)
                                        : f16_gemm_v2_workspace_bytes(batch, n, m, num_cus));
@@ -95,6 +128,15 @@ hipError_t launch_q8_0_gemm(float* y, const uint8_t* w, const float* x, const fl
                             size_t n, size_t m, size_t batch, void* ws, int num_cus,
                             hipStream_t s) {
   uint8_t* base = static_cast<uint8_t*>(ws);
+  const BlockPlan b = q8_0_plan(w, n, m, batch, num_cus);
+  if (b.splits) {
+    hipError_t be = launch_x_f16_onepass(x, batch, m, ws, false, s);
+    if (be != hipSuccess) return be;
+    return launch_block_gemm_f16x(
+        b, kFmtQ8_0, y, w, bias, n, m, batch, ws, (batch + 127) / 128 * 128 * m * 2,
+        gemm_x_exponents(ws, batch, m),
+        reinterpret_cast<float*>(base + round256(gemm_workspace_bytes(batch, m))), s);
+  }
   _Float16* w16 = reinterpret_cast<_Float16*>(base);
   float* D = reinterpret_cast<float*>(base + round256(n * m * 2));
   void* gemm_ws = base + round256(n * m * 2) + round256(n * 4);
