@@ -447,19 +447,20 @@ int q4_0_col_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const
     cus = ds->cus;
   }
   hipError_t e;
-  // Many tokens: the tensor expanded once to fp16 pairs and a GEMM, against
-  // the one-token kernel over groups of tokens.  Measured per call (us, old
-  // and new): 2048 x 2048 15.7 / 20.4 at 8 tokens, 42.7 / 22.8 at 32, 139 /
-  // 31.8 at 128; 5632 x 2048 19.5 / 31.5 at 4, 54.1 / 30.7 at 16, 399 / 40.6
-  // at 128; 14336 x 4096 104 / 106 at 16, 201 / 108 at 32; 512 x 544 16.8 /
-  // 17.0 at 64: about 5 us and 0.25 us per million weights and token (0.11
-  // beyond 32M, which fill the chip) against 15 us, 1.45 us per million
-  // weights and 0.025 per million and token.  Up to 512 MB of expansion.
+  // Several tokens: the pair GEMM, against the one-token kernel over groups of
+  // tokens.  Measured per call (us, one-token kernel and GEMM): 2048 x 2048
+  // 16 / 17.2 at 8, 26.4 / 17.5 at 16, 144 / 20.5 at 128; 5632 x 2048 31 / 17.5
+  // at 8, 52 / 17 at 16, 412 / 28 at 128; 14336 x 4096 52 / 28 at 8, 2885 / 174
+  // at 512; 1024 x 512 14.7 / 17 at 16, 19.4 / 17 at 64: about
+  // 8 us and 0.25 us per million weights and token (0.11 beyond 32M, which
+  // fill the chip) against 17 us (three launches), 0.17 us per million weights
+  // and 0.006 per million and token.  Fewer than 8 tokens stay with the
+  // one-token kernel, whose rows equal one-token calls bit for bit.
   {
     const double mw = (double)n * m * 1e-6;
-    const double one = 5.0 + batch * mw * (mw < 32.0 ? 0.25 : 0.11);
-    const double many = 15.0 + mw * (1.45 + 0.025 * batch);
-    if (batch > 1 && many < one && mw <= 128.0 && q4_0_col_gemm_ok(w, w_len, n, m, batch)) {
+    const double one = 8.0 + batch * mw * (mw < 32.0 ? 0.25 : 0.11);
+    const double many = 17.0 + mw * (0.17 + 0.006 * batch);
+    if (batch >= 8 && many < one && q4_0_col_gemm_ok(w, w_len, n, m, batch)) {
       const size_t bytes = q4_0_col_gemm_workspace_bytes(n, m, batch, cus);
       if (workspace_can_hold(ds, s, bytes)) {
         WsLock ws;

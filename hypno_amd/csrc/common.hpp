@@ -416,8 +416,7 @@ hipError_t launch_split_reduce(float* y, const float* part, const float* bias, s
                                int splits, hipStream_t s);
 
 // fp32-accurate batched GEMMs on fp16 operand pairs (gemm_pair.hip):
-// column-major Q4_0 expanded once per call, and fp16 weights with any
-// m % 32 == 0.
+// column-major Q4_0, and fp16 weights with any m % 32 == 0.
 bool q4_0_col_gemm_ok(const uint8_t* w, size_t w_len, size_t n, size_t m, size_t batch);
 size_t q4_0_col_gemm_workspace_bytes(size_t n, size_t m, size_t batch, int num_cus);
 hipError_t launch_q4_0_col_gemm(float* y, const uint8_t* w, size_t w_len, const float* x,

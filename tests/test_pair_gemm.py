@@ -32,7 +32,8 @@ def _col(torch, wb, x, bias, n, m):
 @pytest.mark.parametrize("tokens,n,m,cut", [(40, 2080, 2080, 0), (33, 3104, 1056, 0),
                                             (65, 1056, 1120, 0), (129, 1024, 1024, 18),
                                             (128, 256, 2048, 0), (300, 544, 1056, 0),
-                                            (64, 1056, 1056, 18 * 33 * 100 + 7)])
+                                            (64, 1056, 1056, 18 * 33 * 100 + 7),
+                                            (8, 5664, 2080, 0), (300, 14336, 544, 18 * 448 * 3)])
 def test_col_major_many_tokens(orc, tokens, n, m, cut):
     import torch
     print(f"col tokens={tokens} n={n} m={m} cut={cut}", flush=True)
