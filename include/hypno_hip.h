@@ -23,6 +23,10 @@
  *         value), products with the nibbles are exact in int32, each block's
  *         sum is scaled by d in fp32 and blocks accumulate in fp32.  Other
  *         shapes: fp32 FMAs.  Bar: max|y - r| / max|r| <= 1e-4.
+ *       Q4_0 and Q8_0 batches whose rows suit none of the kernels below
+ *         (m % 32 == 0): fp16 hi/lo activation pairs per token (to ~2^-22),
+ *         exact integer products on MFMA, block scale in fp32, from 80M
+ *         products; fewer take fp32 FMAs token by token.
  *       Q4_0, M = 2 (M <= 4 when n * m <= 16M),
  *         m % 256 == 0: the
  *         streaming GEMV with every block multiplied by each token's row, in
@@ -44,11 +48,15 @@
  *         lo (x 2^s = hi + lo to ~2^-22), on MFMA against the fp16 weights
  *         with fp32 accumulation (the 1e-4 bar per token; fp32 FMAs token by
  *         token if x is not 16-byte aligned); M >= 16 as the Q4_0 GEMM with
- *         fp16 weights.
+ *         fp16 weights.  Rows of m % 64 == 32: hi and lo rows at every M.
  *       Q8_0: M < 16 each token's activations as three exact int8 digit
  *         planes per block (to 2^-23), each weight block read once for 2 to 8
- *         tokens; M >= 16 weights expanded once to fp16 (row-normalised,
- *         relative 2^-11) and the FP16 GEMM.
+ *         tokens; M >= 16 as the Q4_0 GEMM with exact integer weights, or
+ *         where that is faster weights expanded once to fp16
+ *         (row-normalised, relative 2^-11) and the FP16 GEMM.
+ *       Column-major Q4_0: fp32 FMAs token by token; from 8 tokens, where it
+ *         is faster, exact fp16 pairs of weights times hi/lo pairs of
+ *         activations on MFMA (the same 1e-4 bar per token).
  *   - Every function returns a status (HYPNO_HIP_OK on success) and never
  *     aborts the process.  hypno_hip_last_error() describes the last failure
  *     on the calling thread.
@@ -198,7 +206,9 @@ int hypno_hip_matmul_q4_0_dev_noalloc(float* y, const uint8_t* w_q, size_t w_len
 
 /* Column-major Q4_0 on device pointers (semantics of
  * hypno_hip_matmul_q4_0_col; batch > 1: each token's product as
- * turbo.rs:322-326 computes it token by token, the tokens run in groups). */
+ * turbo.rs:322-326 computes it token by token.  Fewer than 8 tokens run in
+ * groups, each row bit-identical to its one-token call; from 8, where it is
+ * faster, the weights are read once for all by an fp32-accurate MFMA GEMM). */
 int hypno_hip_matmul_q4_0_col_dev(float* y, const uint8_t* w_q, size_t w_len, const float* x,
                                   const float* bias, size_t n, size_t m, size_t batch,
                                   void* stream);
@@ -210,10 +220,11 @@ int hypno_hip_matmul_f16_dev(float* y, const uint8_t* w, size_t w_len, const flo
 
 /* Q8_0 on device pointers (ops.rs:33-36 for batch == 1; turbo.rs:334-341
  * semantics for batch > 1).  batch >= 16 with m % 64 == 0 runs a prefill
- * GEMM on an fp16 expansion of the weights (rel-L2 <= 2e-3 of the exact
- * product); smaller batches (m % 256 == 0, x 16-byte aligned) read each
+ * GEMM on the blocks or on an fp16 expansion of the weights, whichever a cost
+ * model has faster (rel-L2 <= 2e-3 of the exact product); smaller batches (m % 256 == 0, x 16-byte aligned) read each
  * weight block once per 2 to 8 tokens, every token's row bit-identical to
- * its one-token call (normwise <= 1e-4); other shapes run token by token. */
+ * its one-token call (normwise <= 1e-4); other shapes run an fp32-accurate
+ * MFMA GEMM from 80M products (m % 32 == 0), token by token below. */
 int hypno_hip_matmul_q8_0_dev(float* y, const uint8_t* w_q, size_t w_len, const float* x,
                               const float* bias, size_t n, size_t m, size_t batch,
                               void* stream);
