@@ -106,13 +106,48 @@ rms_norm_rows_vec_kernel(float* out, const float* x, const float* __restrict__ w
   }
 }
 
+__device__ __forceinline__ float silu(float g) { return g / (1.0f + expf(-g)); }
+
 __global__ void __launch_bounds__(256)
 silu_mul_kernel(float* out, const float* gate, const float* __restrict__ up, size_t n) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x) {
-    const float g = gate[i];
-    out[i] = g / (1.0f + expf(-g)) * up[i];
+    out[i] = silu(gate[i]) * up[i];
   }
+}
+
+// The same on 16-byte vectors, kSiluVecs of gate and of up per thread in flight
+// together; the last n % 4 elements one a thread.  Every vector is read before
+// its place is written, so out may be gate or up.  Bound by HBM (by the launch
+// for a few tokens): a 4-byte load a thread per grid step kept too few bytes in
+// flight.  Per launch, before -> after: 2048 x 14336 68.0 -> 64.8 us (5.4 TB/s),
+// 512 x 14336 14.9 -> 14.0, 333 x 7200 8.2 -> 7.6; one vector a thread 64.2,
+// 14.3 and 7.7, four 65.8, 14.4 and 7.8.
+constexpr int kSiluVecs = 2;
+__global__ void __launch_bounds__(256)
+silu_mul_vec_kernel(float* out, const float* gate, const float* up, size_t n) {
+  const size_t nv = n / 4;
+  const float4* gv = reinterpret_cast<const float4*>(gate);
+  const float4* uv = reinterpret_cast<const float4*>(up);
+  const size_t first = (size_t)blockIdx.x * (256 * kSiluVecs) + threadIdx.x;
+  float4 g[kSiluVecs], v[kSiluVecs];
+#pragma unroll
+  for (int k = 0; k < kSiluVecs; k++) {
+    const size_t i = first + k * 256;
+    const size_t j = i < nv ? i : 0;
+    g[k] = load_global<float4>(gv + j);
+    v[k] = load_global<float4>(uv + j);
+  }
+#pragma unroll
+  for (int k = 0; k < kSiluVecs; k++) {
+    const size_t i = first + k * 256;
+    if (i >= nv) break;
+    reinterpret_cast<float4*>(out)[i] =
+        make_float4(silu(g[k].x) * v[k].x, silu(g[k].y) * v[k].y, silu(g[k].z) * v[k].z,
+                    silu(g[k].w) * v[k].w);
+  }
+  const size_t e = 4 * nv + threadIdx.x;
+  if (blockIdx.x == 0 && e < n) out[e] = silu(gate[e]) * up[e];
 }
 
 }  // namespace
@@ -142,6 +177,13 @@ hipError_t launch_rms_norm(float* out, const float* x, const float* weight, size
 hipError_t launch_silu_mul(float* out, const float* gate, const float* up, size_t n,
                            hipStream_t s) {
   if (n == 0) return hipSuccess;
+  const size_t groups = (n / 4 + 256 * kSiluVecs - 1) / (256 * kSiluVecs);
+  if (n >= 4 && groups <= 0xFFFFFF &&
+      (((uintptr_t)out | (uintptr_t)gate | (uintptr_t)up) & 15) == 0) {
+    hipLaunchKernelGGL(silu_mul_vec_kernel, dim3((unsigned)groups), dim3(256), 0, s, out, gate, up,
+                       n);
+    return hipGetLastError();
+  }
   size_t grid = (n + 255) / 256;
   if (grid > 4096) grid = 4096;
   hipLaunchKernelGGL(silu_mul_kernel, dim3((unsigned)grid), dim3(256), 0, s, out, gate, up, n);
