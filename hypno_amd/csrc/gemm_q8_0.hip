@@ -99,7 +99,7 @@ bool q8_0_use_stream(size_t n, size_t m, size_t batch) {
 // The block GEMM's plan, or splits = 0 where the expanded weights are faster:
 // from one work-group of 128 x 256 per CU that way costs about 3 + 0.62 us per
 // million weights to expand and, a round, 3 + 1.1 us per 64 columns of K.  Up
-// to 64 MB of partial planes (the expansion needs more than that anyway).
+// to 64 MB of partial planes (what the expansion of 32M weights takes).
 static BlockPlan q8_0_plan(const uint8_t* w, size_t n, size_t m, size_t batch, int num_cus) {
   const size_t bytes = n * (m / kBlockElems) * kQ8BlockBytes;
   if (!block_gemm_ok(kFmtQ8_0, w, bytes, n, m, batch)) return BlockPlan{0, 0, 0.0};
