@@ -484,8 +484,13 @@ x_rows_block_kernel(u32x4* __restrict__ xh, int* __restrict__ xexp, const float*
     u32x4 a, b;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-      const float s0 = ldexpf(e[kPerm ? perm[2 * j] : 2 * j], sh);
-      const float s1 = ldexpf(e[kPerm ? perm[2 * j + 1] : 2 * j + 1], sh);
+      // (a finite value past fp16's range, which only a row without a scale of
+      // its own can hold, stays finite: that row's outputs are the infinity's)
+      auto in_range = [](float f) {
+        return fabsf(f) < __builtin_inff() ? fminf(fmaxf(f, -65504.0f), 65504.0f) : f;
+      };
+      const float s0 = in_range(ldexpf(e[kPerm ? perm[2 * j] : 2 * j], sh));
+      const float s1 = in_range(ldexpf(e[kPerm ? perm[2 * j + 1] : 2 * j + 1], sh));
       const _Float16 h0 = (_Float16)s0, h1 = (_Float16)s1;
       a[j] = (uint32_t)__builtin_bit_cast(uint16_t, h0) |
              ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
