@@ -336,11 +336,22 @@ __global__ void __launch_bounds__(kPThreads, 1) gemm_pair_kernel(const PairArgs 
     }
     return v;
   };
+  // The same from fp16 rows: where the pairs' sum is NaN, which an infinity (in
+  // the weights or the token) makes of finite neighbours (inf times a zero or
+  // an opposite lo part).
+  auto from_rows = [&](int m) -> float {
+    float v = 0.0f;
+    const int k1 = min(a.K, s1 * kPStageK);
+    const uint16_t* w = reinterpret_cast<const uint16_t*>(a.wh) + (size_t)ncol * a.K;
+    for (int k = s0 * kPStageK; k < k1; k++)
+      v = fmaf(f16_bits_to_f32(w[k]), a.x[(size_t)m * a.K + k], v);
+    return v;
+  };
   const bool big = kCol && __any(dmax > kBigScale);
 #pragma unroll
   for (int i = 0; i < MT; i++) {
     uint32_t ex[16];
-    bool odd_row = big;
+    uint32_t redo = big ? 0xFFFFu : 0u;  // registers to compute from the source
 #pragma unroll
     for (int r = 0; r < 16; r++) {
       ex[r] = __builtin_amdgcn_raw_buffer_load_b32(
@@ -350,15 +361,15 @@ __global__ void __launch_bounds__(kPThreads, 1) gemm_pair_kernel(const PairArgs 
     for (int r = 0; r < 16; r++) {
       const uint32_t m = (uint32_t)(m0 + 32 * i + 8 * (r / 4) + 4 * h + r % 4);
       const uint32_t off = nvalid ? (m * (uint32_t)a.N + (uint32_t)ncol) * 4u : 0xFFFFFFF0u;
-      if (kCol) odd_row = odd_row || ex[r] == kNotFinite;
+      if (kCol ? ex[r] == kNotFinite : acc[i][r] != acc[i][r]) redo |= 1u << r;
       const float v = ldexpf(acc[i][r], (int)ex[r]) + bv;
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), yrs, off, 0, 0);
     }
-    if (kCol && odd_row && nvalid) {
+    if (redo && nvalid) {
       for (int r = 0; r < 16; r++) {
         const int m = m0 + 32 * i + 8 * (r / 4) + 4 * h + r % 4;
-        if (m < a.M && (big || (uint32_t)a.xexp[m] == kNotFinite))
-          dst[(size_t)m * a.N + ncol] = from_blocks(m) + bv;
+        if (m < a.M && (redo >> r & 1))
+          dst[(size_t)m * a.N + ncol] = (kCol ? from_blocks(m) : from_rows(m)) + bv;
       }
     }
   }

@@ -60,3 +60,27 @@ def test_block_batch(orc, dt, tokens, n, m):
     x = _tokens(rng, tokens, m)
     got = _run(torch, f"hypno_hip_matmul_{dt}_dev", wb, x, n, m)
     _check(orc, got, x, w[:n * m].reshape(n, m).astype(np.float64))
+
+
+@pytest.mark.parametrize("tokens,n,m", [(8, 300, 1056), (70, 520, 2080)])
+def test_f16_batch(orc, tokens, n, m):
+    """fp16 rows of K % 64 == 32, finite and with infinite weights in columns
+    where tokens hold values that fp16 has exactly (a zero lo part) and not."""
+    import torch
+    print(f"f16 tokens={tokens} n={n} m={m}", flush=True)
+    rng = np.random.default_rng(n + m)
+    w = (rng.standard_normal((n, m)) * 0.02).astype(np.float16)
+    x = _tokens(rng, tokens, m)
+    x[5, 33], x[6, 33], x[7, 33] = 1.0, -2.5, 0.0
+    fn = "hypno_hip_matmul_f16_dev"
+    _check(orc, _run(torch, fn, w.ravel().view(np.uint8), x, n, m), x, w.astype(np.float64))
+    inf = {3: (33, np.inf), n // 2: (33, -np.inf), n - 1: (m - 1, np.inf)}
+    for r, (k, v) in inf.items():
+        w[r, k] = v
+    got = _run(torch, fn, w.ravel().view(np.uint8), x, n, m)
+    one = np.concatenate([_run(torch, fn, w.ravel().view(np.uint8), x[t:t + 1], n, m)
+                          for t in range(tokens)])  # the one-token product: fp32 FMAs
+    for r in inf:
+        assert np.array_equal(got[:, r], one[:, r], equal_nan=True), r
+    rest = np.setdiff1d(np.arange(n), list(inf))
+    _check(orc, got[:, rest], x, w[rest].astype(np.float64))
