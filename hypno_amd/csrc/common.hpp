@@ -406,6 +406,11 @@ hipError_t launch_block_gemm_f16x(const BlockPlan& p, int fmt, float* y, const u
                                   const void* xh, size_t x_bytes, const int* xexp, float* part,
                                   hipStream_t s);
 
+// X fp32 [batch][m] -> three bf16 planes [batch][kp] (kp: m in whole 64s) that
+// hold x 2^s exactly, then the rows' exponents (gemm_block.hip).
+size_t x_split_bytes(size_t batch, size_t m);
+int* x_split_exponents(void* xs, size_t batch, size_t m);
+hipError_t launch_x_split(void* xs, const float* x, size_t batch, size_t m, hipStream_t s);
 // X fp32 [batch][m] -> fp16 [batch][kp] hi parts and a plane of lo parts in
 // natural column order, per-row exponents at xexp; with `clear`, *clear = 0
 // and the exponent of a row holding inf or NaN is INT_MIN.

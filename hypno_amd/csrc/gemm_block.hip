@@ -5,25 +5,27 @@
 // which the alternative is one fp32 dot product per token and row.
 //
 // Arithmetic: the integer weights (nibble - 8, or byte - 128) go to the
-// matrix cores as exact fp16 values.  Each token is two fp16 rows, hi and lo
-// (x 2^s = hi + lo to ~2^-22, s a power of two per token undone exactly on
-// output), whose products with a block add up in one partial P (K = 32: four
-// chained v_mfma_f32_32x32x16_f16 from a zeroed accumulator); the block's d
-// scales it in fp32, acc += d * P.
+// matrix cores as exact bf16 values.  Each token is three bf16 rows that hold
+// all 24 bits of x (x 2^s = x1 + x2 + x3, each the next 8 bits; s a power of
+// two per token that keeps every sum in range, undone exactly on output),
+// whose products with a block, all exact, add up smallest first in one partial
+// P (K = 32: six chained v_mfma_f32_32x32x16_bf16 from a zeroed accumulator);
+// the block's d scales it in fp32, acc += d * P.
 //
 // What bounds it: the 16 scale FMAs per 32 x 32 output tile and block share
 // the SIMD's issue port with the MFMAs, and every wave reads the whole X tile
 // from LDS.  The 32x32x16 form issues half as many MFMAs per product as
 // 16x16x32 and an A operand feeds 32 columns.  Measured: 333 tokens, N 2880,
-// K 7200 (225 blocks a row): 57 us per call where the fp32 dot products took
-// 14.5 ms; rel-L2 against them 2.4e-7.
+// K 7200 (225 blocks a row): 74-81 us per call where the fp32 dot products took
+// 14.5 ms, error against 64 bits 1.4e-7 (1.9e-7).  With two fp16 parts in place
+// of three bf16 ones (60 us) x keeps 22 bits, fewer beside an outlier.
 //
 //  * Work-group = 8 waves (two per SIMD) on a 32 MT x 256 tile of Y; wave w
 //    owns output columns 32 w .. 32 w + 31 for all 32 MT rows.  Its weights
 //    reach its own LDS ring by DMA (4 bytes per lane; only the wave's own
 //    load counter orders that ring) and are unpacked in registers, once per
 //    block for MT tiles of rows.
-//  * X: fp16 rows by DMA into a ring of kRing stages of 64 K shared by the
+//  * X: 16-bit rows by DMA into a ring of kRing stages of 64 K shared by the
 //    waves, 16-byte chunk c of row r in slot c ^ ((r >> 1) & 7) (16 rows of
 //    an operand read hit distinct banks).  One barrier per stage: it
 //    publishes the stage two ahead.
@@ -32,7 +34,7 @@
 //    j + 2, the 16 scale FMAs of slot j - 1 and a share of the next block's
 //    unpack, in that order (a scheduling barrier between slots).
 //  * One part: x rounded once to fp16 (the prefill GEMMs' arithmetic) takes
-//    the same kernel without the lo rows, half the MFMAs and half the LDS per
+//    the same kernel on fp16 operands, a third of the MFMAs and of the LDS per
 //    row, so tiles go up to 256 rows.  Per 256 x 256 x 64 stage 2.3 us with
 //    every CU at work (930 TFLOP/s); copies without X and W DMA 13% faster,
 //    without the barrier 4%, without the A reads no faster: what is left is
@@ -51,6 +53,7 @@ namespace hypno {
 namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kBWaves = 8;
@@ -61,18 +64,18 @@ constexpr int kBRowBytes = kBStageK * 2;
 
 // FMT: weight format; MT: 32-row tiles per wave; ODD: an odd number of blocks
 // per row.
-template <int FMT, int MT, bool ODD, int PARTS = 2>
+template <int FMT, int MT, bool ODD, int PARTS = 3>
 struct BlockGeom {
   static constexpr int kBlk = FMT == kFmtQ8_0 ? kQ8BlockBytes : kBlockBytes;
   static constexpr int kRowDw = 2 * kBlk / 4 + (ODD ? 1 : 0);  // a row's dwords per stage
   static constexpr int kDw = (32 * kRowDw + 63) / 64;          // W DMAs per wave and stage
   static constexpr int kWSlot = 256 * kDw;
-  static constexpr int kXRows = 32 * PARTS * MT;  // hi rows, then lo rows
+  // X rows of the tile, part by part (padded to whole DMAs of every wave)
+  static constexpr int kXRows = (32 * PARTS * MT + 63) / 64 * 64;
   static constexpr int kTile = kXRows * kBRowBytes;
   static constexpr int kDx = kXRows / 64;  // X DMAs per wave and stage
-  static_assert(kXRows % 64 == 0, "every wave issues the same number of X DMAs");
   static constexpr int kFree = 160 * 1024;
-  static constexpr int kRing = kTile >= 32768 ? 3 : 4;
+  static constexpr int kRing = kTile >= 24576 ? 3 : 4;
   static constexpr int kFit = (kFree - kRing * kTile) / (kBWaves * kWSlot);
   static constexpr int kMost = FMT == kFmtQ8_0 ? 4 : 6;  // (vmcnt counts to 63)
   static constexpr int kWRing = kFit > kMost ? kMost : kFit;
@@ -88,7 +91,7 @@ struct BlockGeom {
 struct BlockArgs {
   float* y;
   const uint8_t* w;
-  const uint8_t* xh;  // fp16 [M][Kp] hi parts, then a plane of M rows of lo parts
+  const uint8_t* xh;  // 16-bit [M][Kp], a plane of M rows per part
   const float* bias;
   const int* xexp;    // [M]: row m of xh holds X row m times 2^-xexp[m]
   float* part;        // [splits][M][N] partial planes (splits > 1)
@@ -107,6 +110,48 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t brsrc(const void* base, uint32
                                            0x00020000);
 }
 
+// The matrix product of one operand pair: fp16 where x is rounded to one part,
+// bf16 where it is three.
+template <int PARTS>
+__device__ __forceinline__ floatx16 block_mfma(u32x4 a, u32x4 b, floatx16 c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (PARTS == 1)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a),
+                                                  __builtin_bit_cast(half8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+#else
+  return c;
+#endif
+}
+
+// Eight packed integers -> eight exact bf16 values in order.  Q4_0: (nibble -
+// 8) / 16, what v_cvt_off_f32_i4 makes of a nibble with its top bit flipped;
+// the caller's scale carries the 16.  Q8_0: byte - 128.
+__device__ __forceinline__ u32x4 unpack8_bf16(uint32_t q) {
+  const uint32_t lo = q ^ 0x88888888u, hi = lo >> 4;
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const uint32_t a = __float_as_uint(__builtin_amdgcn_cvt_off_f32_i4(lo >> (8 * i)));
+    const uint32_t b = __float_as_uint(__builtin_amdgcn_cvt_off_f32_i4(hi >> (8 * i)));
+    r[i] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+  }
+  return r;
+}
+__device__ __forceinline__ u32x4 unpack8_bytes_bf16(uint32_t lo, uint32_t hi) {
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const uint32_t s = (i < 2 ? lo : hi) ^ 0x80808080u;
+    const uint32_t a = __float_as_uint((float)(int8_t)(s >> (16 * (i & 1))));
+    const uint32_t b = __float_as_uint((float)(int8_t)(s >> (16 * (i & 1) + 8)));
+    r[i] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+  }
+  return r;
+}
+
 // One lane's weights of a block: the integers its two B operands hold (lane
 // half h takes elements 16 h + 8 j .. + 7 for MFMA j), packed, and the scale
 // bits.
@@ -122,7 +167,7 @@ __global__ void __launch_bounds__(kBThreads, 1) gemm_block_kernel(const BlockArg
   using G = BlockGeom<FMT, MT, ODD, PARTS>;
   constexpr int BM = 32 * MT;
   constexpr int kRing = G::kRing, kWRing = G::kWRing;
-  constexpr int kParts = PARTS;  // hi, lo; or the rounded x alone
+  constexpr int kParts = PARTS;  // x1, x2, x3; or the rounded x alone
   extern __shared__ __align__(16) uint8_t smem[];
   const int t = threadIdx.x;
   const int lane = t & 63;
@@ -145,12 +190,10 @@ __global__ void __launch_bounds__(kBThreads, 1) gemm_block_kernel(const BlockArg
   const int steps = s1 - s0;
 
   // --- X DMA: instruction i of wave w fills LDS rows 8 (8 i + w) .. + 7 of
-  // the slot (rows BM .. 2 BM - 1 are the lo parts); lane -> row
+  // the slot (part p in rows BM p .. BM p + BM - 1); lane -> row
   // 8 (8 i + w) + (lane >> 3), slot chunk lane & 7, which holds logical chunk
   // (lane & 7) ^ ((row >> 1) & 7).
   const uint32_t x_row = (uint32_t)a.steps * kBRowBytes;
-  const __amdgpu_buffer_rsrc_t xrs = brsrc(a.xh, a.x_bytes);
-  const __amdgpu_buffer_rsrc_t xls = brsrc(a.xh + a.x_bytes, a.x_bytes);
   uint32_t xvoff[G::kDx];
 #pragma unroll
   for (int i = 0; i < G::kDx; i++) {
@@ -165,9 +208,10 @@ __global__ void __launch_bounds__(kBThreads, 1) gemm_block_kernel(const BlockArg
     uint8_t* slot = smem + (s % kRing) * G::kTile;
 #pragma unroll
     for (int i = 0; i < G::kDx; i++) {
-      const bool lo = PARTS == 2 && 8 * (8 * i + wave) >= BM;  // wave-uniform
+      // (wave-uniform; rows that only fill up the last DMA read the last part again)
+      const int part = min(8 * (8 * i + wave) / BM, PARTS - 1);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          lo ? xls : xrs,
+          brsrc(a.xh + (size_t)part * a.x_bytes, a.x_bytes),
           (__attribute__((address_space(3))) void*)(slot + 8 * (8 * i + wave) * kBRowBytes), 16,
           xvoff[i], soff, 0, 0);
     }
@@ -245,20 +289,22 @@ __global__ void __launch_bounds__(kBThreads, 1) gemm_block_kernel(const BlockArg
       o.d = kb == 0 ? w.d & 0xFFFFu : w.d >> 16;
     }
   };
-  auto unpack = [&](const RawBlock<FMT>& o, int j) __attribute__((always_inline)) -> half8 {
+  auto unpack = [&](const RawBlock<FMT>& o, int j) __attribute__((always_inline)) -> u32x4 {
     if constexpr (FMT == kFmtQ8_0)
-      return __builtin_bit_cast(half8, unpack8_bytes(o.q[2 * j], o.q[2 * j + 1]));
+      return PARTS == 1 ? unpack8_bytes(o.q[2 * j], o.q[2 * j + 1])
+                        : unpack8_bytes_bf16(o.q[2 * j], o.q[2 * j + 1]);
     else
-      return __builtin_bit_cast(half8, unpack8(o.q[j]));
+      return PARTS == 1 ? unpack8(o.q[j]) : unpack8_bf16(o.q[j]);
   };
   // A block past the row's end (K % 64 == 32, block 1 of the last stage)
   // multiplies X's zero padding; its scale bits are not the row's: take 0.
   auto scale_of = [&](const RawBlock<FMT>& o, int s, int kb) __attribute__((always_inline)) {
     const bool ok = nvalid && (!ODD || kb == 0 || 2 * (s0 + s) + 1 < a.B);
-    return ok ? f16_bits_to_f32(o.d) : 0.0f;
+    const float unit = FMT == kFmtQ4_0 && PARTS == 3 ? 16.0f : 1.0f;
+    return ok ? f16_bits_to_f32(o.d) * unit : 0.0f;
   };
 
-  // --- A operands: part p (hi, lo), block kb, MFMA j, row tile i: row
+  // --- A operands: part p, block kb, MFMA j, row tile i: row
   // 32 i + lr (+ BM p), logical chunk 4 kb + 2 h + j.
   uint32_t aoff[2][2];
 #pragma unroll
@@ -266,8 +312,8 @@ __global__ void __launch_bounds__(kBThreads, 1) gemm_block_kernel(const BlockArg
 #pragma unroll
     for (int j = 0; j < 2; j++)
       aoff[kb][j] = (uint32_t)lr * kBRowBytes + (((4 * kb + 2 * h + j) ^ ((lr >> 1) & 7)) << 4);
-  auto read_a = [&](int s, int kb, int i, int p, int j) __attribute__((always_inline)) -> half8 {
-    return *reinterpret_cast<const half8*>(smem + (s % kRing) * G::kTile + aoff[kb][j] +
+  auto read_a = [&](int s, int kb, int i, int p, int j) __attribute__((always_inline)) -> u32x4 {
+    return *reinterpret_cast<const u32x4*>(smem + (s % kRing) * G::kTile + aoff[kb][j] +
                                            (32 * i + BM * p) * kBRowBytes);
   };
 
@@ -276,6 +322,18 @@ __global__ void __launch_bounds__(kBThreads, 1) gemm_block_kernel(const BlockArg
   for (int i = 0; i < MT; i++)
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[i][r] = 0.0f;
+  // Three parts: the sum moves to `tot` every kGroup stages, so no output is a
+  // chain of one rounding per block (1000 tokens, K 2848 in one piece: rel-L2
+  // 1.8e-7 as one chain, 1.0e-7 so, 1.4e-7 the fp32 dot products).
+  constexpr int kGroup = 8;
+  constexpr int kTot = PARTS == 3 ? MT : 1;
+  floatx16 tot[kTot];
+  if constexpr (PARTS == 3) {
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) tot[i][r] = 0.0f;
+  }
 
   // Prologue: X of stages 0..R-2 and W of stages 0..P-1 in flight; X and W of
   // stages 0 and 1 landed and published; the A operands of slots 0 and 1 and
@@ -284,14 +342,14 @@ __global__ void __launch_bounds__(kBThreads, 1) gemm_block_kernel(const BlockArg
   for (int i = 0; i < kWRing; i++) issue_w(i);
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(G::kDw * (kWRing - 2)) : "memory");
   constexpr int kSlots = 2 * MT;
-  half8 fa[2][kParts][2];  // slot j's operands: fa[j & 1]
+  u32x4 fa[2][kParts][2];  // slot j's operands: fa[j & 1]
 #pragma unroll
   for (int j = 0; j < 2; j++)
 #pragma unroll
     for (int p = 0; p < kParts; p++)
 #pragma unroll
       for (int k = 0; k < 2; k++) fa[j][p][k] = read_a(0, j / MT, j % MT, p, k);
-  half8 fb[2];
+  u32x4 fb[2];
   float d;
   Win wodd = read_win(0, 1);
   {
@@ -309,7 +367,7 @@ __global__ void __launch_bounds__(kBThreads, 1) gemm_block_kernel(const BlockArg
   for (int s = 0; s < steps; s++) {
     const Win weven = read_win(s + 1, 0);
     Win wodd_next = wodd;
-    half8 nb[2];
+    u32x4 nb[2];
     float nd = 0.0f;
     RawBlock<FMT> raw;
 #pragma unroll
@@ -327,10 +385,9 @@ __global__ void __launch_bounds__(kBThreads, 1) gemm_block_kernel(const BlockArg
 #pragma unroll
       for (int r = 0; r < 16; r++) p[r] = 0.0f;
 #pragma unroll
-      for (int q = 0; q < kParts; q++)
+      for (int q = kParts - 1; q >= 0; q--)  // the smallest parts first
 #pragma unroll
-        for (int k = 0; k < 2; k++)
-          p = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[j & 1][q][k], fb[k], p, 0, 0, 0);
+        for (int k = 0; k < 2; k++) p = block_mfma<PARTS>(fa[j & 1][q][k], fb[k], p);
       // operands of slot j + 2
       {
         const int nj = j + 2;
@@ -370,11 +427,28 @@ __global__ void __launch_bounds__(kBThreads, 1) gemm_block_kernel(const BlockArg
       }
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (PARTS == 3) {
+      if (s % kGroup == kGroup - 1) {
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) {
+            tot[i][r] += acc[i][r];
+            acc[i][r] = 0.0f;
+          }
+      }
+    }
     wodd = wodd_next;
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(G::kStageWait) : "memory");
   }
 #pragma unroll
   for (int r = 0; r < 16; r++) acc[MT - 1][r] = fmaf(dprev, prev[r], acc[MT - 1][r]);
+  if constexpr (PARTS == 3) {
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[i][r] += tot[i][r];
+  }
   // Every DMA into LDS (the trailing re-reads included) has landed before
   // the work-group's LDS is released.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -417,16 +491,114 @@ block_split_reduce_kernel(float* __restrict__ y, const float* __restrict__ part,
   y[i] = v + (bias ? bias[i % n] : 0.0f);
 }
 
+// X fp32 [M][K] -> three bf16 planes [M][Kp], `plane` vectors apart, one
+// work-group of 256 threads per row: x 2^sh = x1 + x2 + x3 exactly, each part
+// the next 8 bits of x with its sign.  sh puts the row's largest finite |x| in
+// [2^(kXTop - 1), 2^kXTop), where no sum of products overflows and the last
+// part of an element is whole down to 2^-186 of that maximum; xexp[row] = -sh,
+// columns K .. Kp - 1 zero.  An infinity or NaN is x1 alone.  The row is read
+// once if it fits the registers (K <= 16384 and 16-byte aligned), twice
+// otherwise.
+constexpr int kXG = 8;
+constexpr int kXTop = 76;
+__global__ void __launch_bounds__(256)
+x_rows_split_kernel(u32x4* __restrict__ xh, int* __restrict__ xexp, const float* __restrict__ x,
+                    size_t plane, int K, int Kp) {
+  __shared__ uint32_t red[4];
+  const int row = blockIdx.x;
+  const int t = threadIdx.x;
+  const int groups = K / 8, gp = Kp / 8;
+  u32x4* dst = xh + (size_t)row * gp;
+  const float* src = x + (size_t)row * K;
+  const bool al = ((uintptr_t)src & 15) == 0;
+  const bool keep = al && groups <= 256 * kXG;
+  float4 v[kXG][2];
+  uint32_t mb = 0;  // largest finite |x| by bit pattern
+  auto load8 = [&](int g, float4& lo, float4& hi) {
+    const float* p = src + (size_t)g * 8;
+    if (al) {
+      lo = load_global<float4>(p);
+      hi = load_global<float4>(p + 4);
+    } else {
+      lo = make_float4(p[0], p[1], p[2], p[3]);
+      hi = make_float4(p[4], p[5], p[6], p[7]);
+    }
+  };
+  auto amax8 = [&](const float4& lo, const float4& hi) {
+    const float e[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const uint32_t b = __float_as_uint(e[i]) & 0x7FFFFFFFu;
+      mb = max(mb, b < 0x7F800000u ? b : 0u);
+    }
+  };
+  if (keep) {
+#pragma unroll
+    for (int u = 0; u < kXG; u++)
+      if (t + 256 * u < groups) load8(t + 256 * u, v[u][0], v[u][1]);
+#pragma unroll
+    for (int u = 0; u < kXG; u++)
+      if (t + 256 * u < groups) amax8(v[u][0], v[u][1]);
+  } else {
+    for (int g = t; g < groups; g += 256) {
+      float4 lo, hi;
+      load8(g, lo, hi);
+      amax8(lo, hi);
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, off, 64));
+  if ((t & 63) == 0) red[t >> 6] = mb;
+  __syncthreads();
+  mb = max(max(red[0], red[1]), max(red[2], red[3]));
+  const int sh = mb ? kXTop - __builtin_amdgcn_frexp_expf(__uint_as_float(mb)) : 0;
+  auto put = [&](int g, const float4& lo, const float4& hi) {
+    const float e[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    uint32_t b[3][8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const float s = ldexpf(e[i], sh);
+      b[0][i] = __float_as_uint(s) & 0xFFFF0000u;
+      const float r1 = s - __uint_as_float(b[0][i]);
+      b[1][i] = __float_as_uint(r1) & 0xFFFF0000u;
+      b[2][i] = __float_as_uint(r1 - __uint_as_float(b[1][i]));
+      if (!(fabsf(s) < __builtin_inff())) {
+        if (s != s) b[0][i] = 0x7FC00000u;
+        b[1][i] = b[2][i] = 0u;
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+      u32x4 o;
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        o[j] = __builtin_amdgcn_perm(b[p][2 * j + 1], b[p][2 * j], 0x07060302u);
+      dst[p * plane + g] = o;
+    }
+  };
+  if (keep) {
+#pragma unroll
+    for (int u = 0; u < kXG; u++)
+      if (t + 256 * u < groups) put(t + 256 * u, v[u][0], v[u][1]);
+  } else {
+    for (int g = t; g < groups; g += 256) {
+      float4 lo, hi;
+      load8(g, lo, hi);
+      put(g, lo, hi);
+    }
+  }
+  if (t < gp - groups)
+    for (int p = 0; p < 3; p++) dst[p * plane + groups + t] = u32x4{0u, 0u, 0u, 0u};
+  if (t == 0) xexp[row] = -sh;
+}
+
 // X fp32 [M][K] -> fp16 [M][Kp] hi parts and, `plane` vectors on, lo parts,
 // one work-group of 256 threads per row: scaled by 2^sh (sh puts the row's
 // largest |x| in [2^14, 2^15); 0 for an all-zero row or one holding inf or
-// NaN), xexp[row] = -sh, columns K .. Kp - 1 zero.  kPerm writes each group
-// of 8 columns in the Q4_0 unpack order e0,e4,e1,e5,e2,e6,e3,e7.  The row is
+// NaN), xexp[row] = -sh, columns K .. Kp - 1 zero.  The row is
 // read once if it fits the registers (K <= 16384 and 16-byte aligned), twice
 // otherwise.  With `clear`, *clear is set to 0 and the exponent of a row
 // holding inf or NaN to INT_MIN.
-constexpr int kXG = 8;
-template <bool kPerm>
 __global__ void __launch_bounds__(256)
 x_rows_block_kernel(u32x4* __restrict__ xh, int* __restrict__ xexp, const float* __restrict__ x,
                     size_t plane, int K, int Kp, uint32_t* __restrict__ clear) {
@@ -480,7 +652,6 @@ x_rows_block_kernel(u32x4* __restrict__ xh, int* __restrict__ xexp, const float*
   if (amax > 0.0f && amax < __builtin_inff()) sh = 15 - __builtin_amdgcn_frexp_expf(amax);
   auto put = [&](int g, const float4& lo, const float4& hi) {
     const float e[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-    constexpr int perm[8] = {0, 4, 1, 5, 2, 6, 3, 7};
     u32x4 a, b;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -489,8 +660,8 @@ x_rows_block_kernel(u32x4* __restrict__ xh, int* __restrict__ xexp, const float*
       auto in_range = [](float f) {
         return fabsf(f) < __builtin_inff() ? fminf(fmaxf(f, -65504.0f), 65504.0f) : f;
       };
-      const float s0 = in_range(ldexpf(e[kPerm ? perm[2 * j] : 2 * j], sh));
-      const float s1 = in_range(ldexpf(e[kPerm ? perm[2 * j + 1] : 2 * j + 1], sh));
+      const float s0 = in_range(ldexpf(e[2 * j], sh));
+      const float s1 = in_range(ldexpf(e[2 * j + 1], sh));
       const _Float16 h0 = (_Float16)s0, h1 = (_Float16)s1;
       a[j] = (uint32_t)__builtin_bit_cast(uint16_t, h0) |
              ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
@@ -528,25 +699,26 @@ size_t rup(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // Geometry chosen for a shape: 32-row tiles per wave and K pieces.
 //
-// Costs (microseconds, measured): a 64-K stage 0.75 / 1.1 / 1.75 on 32- / 64- /
-// 128-row tiles; a round of work-groups
-// (one per CU) ~3 more to fill and drain; K pieces add the reduction launch
-// (~2.5) and its read of every partial plane (~4 TB/s).
+// Costs (microseconds, fitted to 26 shapes at every number of pieces; the plans
+// they choose measured 1.3% above the best on average): a 64-K stage
+// 0.85 / 1.2 on 32- / 64-row tiles, a round of work-groups (one per CU) ~3
+// more to fill and drain; K pieces add the reduction launch (~2.5) and the
+// partial planes' traffic (~2 TB/s a way).
 BlockPlan block_plan(size_t n, size_t m, size_t batch, int num_cus) {
   const size_t tn = (n + kBN - 1) / kBN;
   const size_t steps = rup(m, kBStageK) / kBStageK;
   BlockPlan best{1, 1, 0.0};
   double best_cost = 1e300;
-  for (int mt : {1, 2, 4}) {
+  for (int mt : {1, 2}) {
     if (mt > 1 && (size_t)16 * mt >= batch) break;  // taller tiles than the rows
     const size_t tm = (batch + 32 * mt - 1) / (32 * mt);
     const size_t tiles = tm * tn;
-    const double stage_us = mt == 4 ? 1.75 : mt == 2 ? 1.1 : 0.75;
+    const double stage_us = mt == 2 ? 1.2 : 0.85;
     for (size_t sp = 1; sp <= std::min<size_t>(steps, 64); sp++) {
       const size_t wgs = tiles * sp;
       const size_t rounds = (wgs + num_cus - 1) / num_cus;
       double cost = (double)rounds * ((double)((steps + sp - 1) / sp) * stage_us + 3.0);
-      if (sp > 1) cost += 2.5 + (double)sp * (double)(batch * n * 4) / 4.0e6;
+      if (sp > 1) cost += 2.5 + (double)sp * (double)(batch * n * 4) / 2.0e6;
       if (cost < best_cost * 0.999) {
         best_cost = cost;
         best = BlockPlan{mt, (int)sp, cost};
@@ -601,12 +773,25 @@ bool block_gemm_ok(int fmt, const uint8_t* w, size_t w_len, size_t n, size_t m, 
   return w_len >= wbytes;
 }
 
-static size_t block_x_bytes(size_t batch, size_t m) {
-  return rup(2 * batch * rup(m, kBStageK) * 2, 256) + rup(batch * 4, 256);
+size_t x_split_bytes(size_t batch, size_t m) {
+  return rup(3 * batch * rup(m, kBStageK) * 2, 256) + rup(batch * 4, 256);
+}
+
+int* x_split_exponents(void* xs, size_t batch, size_t m) {
+  return reinterpret_cast<int*>(static_cast<uint8_t*>(xs) +
+                                rup(3 * batch * rup(m, kBStageK) * 2, 256));
+}
+
+hipError_t launch_x_split(void* xs, const float* x, size_t batch, size_t m, hipStream_t s) {
+  const size_t kp = rup(m, kBStageK);
+  hipLaunchKernelGGL(x_rows_split_kernel, dim3((unsigned)batch), dim3(256), 0, s,
+                     static_cast<u32x4*>(xs), x_split_exponents(xs, batch, m), x, batch * kp / 8,
+                     (int)m, (int)kp);
+  return hipGetLastError();
 }
 
 size_t block_gemm_workspace_bytes(const BlockPlan& p, size_t n, size_t m, size_t batch) {
-  return block_x_bytes(batch, m) + (p.splits > 1 ? (size_t)p.splits * batch * n * 4 : 0);
+  return x_split_bytes(batch, m) + (p.splits > 1 ? (size_t)p.splits * batch * n * 4 : 0);
 }
 
 template <int FMT, bool ODD>
@@ -617,9 +802,8 @@ static hipError_t launch_block_mt(const BlockPlan& p, const BlockArgs& a, hipStr
     hipLaunchKernelGGL(kernel, dim3(a.tiles_m * a.tiles_n, p.splits), dim3(kBThreads), lds, s, a);
     return hipGetLastError();
   };
-  if (p.mt == 4) return go(gemm_block_kernel<FMT, 4, ODD, 2>, BlockGeom<FMT, 4, ODD>::kLds);
-  if (p.mt == 2) return go(gemm_block_kernel<FMT, 2, ODD, 2>, BlockGeom<FMT, 2, ODD>::kLds);
-  return go(gemm_block_kernel<FMT, 1, ODD, 2>, BlockGeom<FMT, 1, ODD>::kLds);
+  if (p.mt == 2) return go(gemm_block_kernel<FMT, 2, ODD, 3>, BlockGeom<FMT, 2, ODD>::kLds);
+  return go(gemm_block_kernel<FMT, 1, ODD, 3>, BlockGeom<FMT, 1, ODD>::kLds);
 }
 
 hipError_t launch_block_gemm(const BlockPlan& p, int fmt, float* y, const uint8_t* w,
@@ -631,10 +815,8 @@ hipError_t launch_block_gemm(const BlockPlan& p, int fmt, float* y, const uint8_
   a.w = w;
   a.xh = static_cast<const uint8_t*>(ws);
   a.bias = bias;
-  int* xexp = reinterpret_cast<int*>(static_cast<uint8_t*>(ws) +
-                                     rup(2 * batch * kp * 2, 256));
-  a.xexp = xexp;
-  a.part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + block_x_bytes(batch, m));
+  a.xexp = x_split_exponents(ws, batch, m);
+  a.part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + x_split_bytes(batch, m));
   a.B = (int)(m / kBlockElems);
   a.w_bytes = (uint32_t)rup(n * a.B * (fmt == kFmtQ8_0 ? kQ8BlockBytes : kBlockBytes), 4);
   a.x_bytes = (uint32_t)(batch * kp * 2);
@@ -647,13 +829,8 @@ hipError_t launch_block_gemm(const BlockPlan& p, int fmt, float* y, const uint8_
   a.xcd_map = (a.tiles_m * a.tiles_n) % 8 == 0 ? 1 : 0;
   a.splits = p.splits;
 
-  auto conv = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)batch), dim3(256), 0, s, static_cast<u32x4*>(ws),
-                       xexp, x, batch * kp / 8, (int)m, (int)kp, nullptr);
-    return hipGetLastError();
-  };
   const bool q8 = fmt == kFmtQ8_0, odd = a.B % 2 != 0;
-  hipError_t e = q8 ? conv(x_rows_block_kernel<false>) : conv(x_rows_block_kernel<true>);
+  hipError_t e = launch_x_split(ws, x, batch, m, s);
   if (e != hipSuccess) return e;
   if (q8)
     e = odd ? launch_block_mt<kFmtQ8_0, true>(p, a, s) : launch_block_mt<kFmtQ8_0, false>(p, a, s);
@@ -713,7 +890,7 @@ hipError_t launch_split_reduce(float* y, const float* part, const float* bias, s
 
 hipError_t launch_x_hilo(void* xh, int* xexp, const float* x, size_t batch, size_t m, size_t kp,
                          uint32_t* clear, hipStream_t s) {
-  hipLaunchKernelGGL(x_rows_block_kernel<false>, dim3((unsigned)batch), dim3(256), 0, s,
+  hipLaunchKernelGGL(x_rows_block_kernel, dim3((unsigned)batch), dim3(256), 0, s,
                      static_cast<u32x4*>(xh), xexp, x, batch * kp / 8, (int)m, (int)kp, clear);
   return hipGetLastError();
 }

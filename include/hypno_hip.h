@@ -24,9 +24,9 @@
  *         sum is scaled by d in fp32 and blocks accumulate in fp32.  Other
  *         shapes: fp32 FMAs.  Bar: max|y - r| / max|r| <= 1e-4.
  *       Q4_0 and Q8_0 batches whose rows suit none of the kernels below
- *         (m % 32 == 0): fp16 hi/lo activation pairs per token (to ~2^-22),
- *         exact integer products on MFMA, block scale in fp32, from 80M
- *         products; fewer take fp32 FMAs token by token.
+ *         (m % 32 == 0): each activation as three bf16 parts that hold all its
+ *         24 bits, exact products with the integers on MFMA, block scale in
+ *         fp32, from 80M products; fewer take fp32 FMAs token by token.
  *       Q4_0, M = 2 (M <= 4 when n * m <= 16M),
  *         m % 256 == 0: the
  *         streaming GEMV with every block multiplied by each token's row, in

@@ -98,3 +98,32 @@ def test_any_shape_plan_and_capture(orc):
         torch.cuda.synchronize()
         for t in range(tokens):
             assert orc.normwise_err(y[t].cpu().numpy(), ref[t]) <= 2e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("tokens,n,m", [(8, 7200, 1440), (40, 1100, 2080), (70, 1300, 2080)])
+def test_any_shape_outlier(orc, dt, tokens, n, m):
+    """Tokens whose largest values, 2^12 to 2^100 times the others, stand in
+    columns of zero weights: outputs keep the accuracy of fp32 sums, as if
+    those columns were not there."""
+    import torch
+
+    from hypno_amd import _lib
+    print(f"{dt} tokens={tokens} n={n} m={m}", flush=True)
+    rng = np.random.default_rng(n)
+    w = (rng.standard_normal((n, m)) * 0.02).astype(np.float32)
+    w[:, 96:128] = 0.0  # one block
+    wb = (orc.quantize_q4_0 if dt == "q4_0" else orc.quantize_q8_0)(w.ravel())
+    x = rng.standard_normal((tokens, m)).astype(np.float32)
+    small = x.copy()
+    x[:, 100] = np.ldexp(np.float32(1.0), 12 + np.arange(tokens) * 88 // max(tokens - 1, 1))
+    small[:, 96:128] = 0.0
+    bias = np.zeros(n, np.float32)
+    got = _run(_lib.load(), torch, dt, wb, x, bias, n, m, tokens, 0)
+    ref = np.stack([(orc.matmul_q4_0_f64 if dt == "q4_0" else orc.matmul_q8_0_f64)(
+        wb, small[t], bias, n, m) for t in range(tokens)])
+    # exact products; random rounding of K / 32 block sums and the 32 products of
+    # each stays under 8 2^-24 of the result's norm (measured: about 4 2^-24)
+    for t in range(tokens):
+        assert orc.rel_l2(got[t], ref[t]) <= 8 * 2.0 ** -24, t
