@@ -238,9 +238,10 @@ struct FixedScratch {
 
 // Batches that no tuned kernel takes: the fp32-accurate block GEMM from 80M
 // products on, if its workspace can be had.  Below that one pass per token of
-// the any-length GEMV is as fast (Q4_0, N 2880, K 7200: 13.9 / 18.7 / 29.6 us
-// at 2 / 4 / 8 tokens against 20.3 / 20.3 / 20.7; N 512, K 1056, 8 tokens 4.6
-// against 14.3); the any-shape kernel beside it is slower from a few million.
+// the any-length GEMV is as fast (Q4_0, N 2880, K 7200: 10.6 / 16.0 / 26.0 us
+// at 2 / 4 / 8 tokens against 21.6 / 21.0 / 21.6; N 512, K 1056, 8 tokens 5.1
+// against 15.0; Q8_0, N 7200, K 2880: 17.5 / 31.3 / 55.8 against 17.9 / 18.5 /
+// 18.8); the any-shape kernel beside it is slower from a few million.
 // *done says whether the block GEMM ran; otherwise the caller goes on.
 int try_block_gemm(int fmt, float* y, const uint8_t* w, size_t w_len, const float* x,
                    const float* bias, size_t n, size_t m, size_t batch, hipStream_t s,

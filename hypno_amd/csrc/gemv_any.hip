@@ -3,7 +3,11 @@
 // (so whole blocks per row, on any 2-byte boundary), any x alignment.  fp32
 // throughout, as the any-shape kernel it stands in for: the integer weights
 // as exact fp16 values, widened in the FMAs; each block's dot product times d
-// added to the row's sum.
+// added to the row's sum.  The dot product is four chains of eight FMAs, not
+// one of 32, and for Q8_0, whose any-shape kernel adds single products over 64
+// lanes, chains of four that add up in fp64, as do its rows: errors against 64
+// bits (any-shape kernel, one chain of 32, this) Q4_0 K 1120 1.1e-7, 1.1e-7,
+// 9.0e-8; Q8_0 K 288 8.0e-8, 1.2e-7, 4.9e-8.
 //
 // Bound by HBM.  The any-shape kernel reads single bytes, 18 bytes apart per
 // lane, one dependent block at a time (4096 x 11008: 101 us, 0.25 TB/s).  Here
@@ -12,9 +16,11 @@
 // 4-byte load of the window that starts at the dword at or below it, kDeep
 // steps ahead, and x sits in LDS as [quarter-block][block] vectors, where the
 // lanes' reads of consecutive blocks hit distinct banks and serve all kR rows.
-// Measured per call, any-shape kernel -> this one: Q4_0 4096 x 11008 101 -> 12.0
-// us (2.1 TB/s), 4096 x 2880 30 -> 6.0, 8192 x 28672 552 -> 43.5 (3.0 TB/s);
-// Q8_0 4096 x 11008 85 -> 16.6 (2.9 TB/s).
+// Measured per call, any-shape kernel -> this one: Q4_0 4096 x 11008 98 -> 11.3
+// us (2.2 TB/s), 4096 x 2880 28.5 -> 5.5, 4228 x 20096 217 -> 23.3; Q8_0 4096 x
+// 11008 61.5 -> 17.0 (2.8 TB/s; 16.4 as one chain of 32).
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace hypno {
@@ -30,6 +36,8 @@ struct AnyFmt {
   static constexpr int kBytes = F == kFmtQ8_0 ? kQ8BlockBytes : kBlockBytes;
   static constexpr int kDw = F == kFmtQ8_0 ? 9 : 5;  // window dwords
   static constexpr int kDeep = F == kFmtQ8_0 ? 2 : 3;
+  // Sums of eight products (Q8_0: four) are chains of FMAs; what they add up in.
+  using Sum = std::conditional_t<F == kFmtQ8_0, double, float>;
 };
 
 template <int F>
@@ -46,6 +54,7 @@ gemv_any_kernel(float* __restrict__ y, const uint8_t* __restrict__ w, size_t w_b
 #if defined(__HIP_DEVICE_COMPILE__)  // (the buffer builtins exist only in the device pass)
   using FT = AnyFmt<F>;
   constexpr int kDw = FT::kDw, kDeep = FT::kDeep;
+  using Sum = typename FT::Sum;
   constexpr int kGroups = 64 / L;
   extern __shared__ __align__(16) float4 xs[];  // [8][B]
   y += (size_t)blockIdx.y * y_tok;
@@ -106,18 +115,18 @@ gemv_any_kernel(float* __restrict__ y, const uint8_t* __restrict__ w, size_t w_b
       xs[(i & 7) * B + (i >> 3)] = make_float4(x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]);
   }
   __syncthreads();
-  float acc[kAR];
+  Sum acc[kAR];
 #pragma unroll
-  for (int r = 0; r < kAR; r++) acc[r] = 0.0f;
+  for (int r = 0; r < kAR; r++) acc[r] = 0;
   for (int s0 = 0; s0 < steps; s0 += kDeep) {
 #pragma unroll
     for (int d = 0; d < kDeep; d++) {
       const int s = s0 + d;
       if (s < steps) {
         const int b = min(s * L + l, B - 1);
-        float dot[kAR];
+        Sum dot[kAR];
 #pragma unroll
-        for (int r = 0; r < kAR; r++) dot[r] = 0.0f;
+        for (int r = 0; r < kAR; r++) dot[r] = 0;
 #pragma unroll
         for (int c = 0; c < 4; c++) {  // eight elements at a time
           const float4 p = xs[(2 * c) * B + b], q = xs[(2 * c + 1) * B + b];
@@ -141,7 +150,7 @@ gemv_any_kernel(float* __restrict__ y, const uint8_t* __restrict__ w, size_t w_b
               const uint32_t u = h[i];
               e[i] = __builtin_bit_cast(half2v, u);
             }
-            float a = dot[r];
+            float a = 0.0f;
             if constexpr (F == kFmtQ4_0) {
               a = fmaf((float)e[0][0], p.x, a);
               a = fmaf((float)e[1][0], p.y, a);
@@ -156,12 +165,13 @@ gemv_any_kernel(float* __restrict__ y, const uint8_t* __restrict__ w, size_t w_b
               a = fmaf((float)e[0][1], p.y, a);
               a = fmaf((float)e[1][0], p.z, a);
               a = fmaf((float)e[1][1], p.w, a);
-              a = fmaf((float)e[2][0], q.x, a);
+              dot[r] += (Sum)a;
+              a = (float)e[2][0] * q.x;
               a = fmaf((float)e[2][1], q.y, a);
               a = fmaf((float)e[3][0], q.z, a);
               a = fmaf((float)e[3][1], q.w, a);
             }
-            dot[r] = a;
+            dot[r] += (Sum)a;
           }
         }
 #pragma unroll
@@ -169,7 +179,7 @@ gemv_any_kernel(float* __restrict__ y, const uint8_t* __restrict__ w, size_t w_b
           const bool odd = (off[r] + (uint32_t)s * (uint32_t)(L * FT::kBytes)) & 2;
           const float sc = f16_bits_to_f32(odd ? win[d][r].v[0] >> 16 : win[d][r].v[0] & 0xFFFFu);
           // (a lane past the row's blocks holds zeros, but x may hold inf or NaN)
-          if (s * L + l < B) acc[r] = fmaf(sc, dot[r], acc[r]);
+          if (s * L + l < B) acc[r] = fma((Sum)sc, dot[r], acc[r]);
           win[d][r] = load(s + kDeep, r);
         }
       }
@@ -177,11 +187,11 @@ gemv_any_kernel(float* __restrict__ y, const uint8_t* __restrict__ w, size_t w_b
   }
 #pragma unroll
   for (int r = 0; r < kAR; r++) {
-    float v = acc[r];
+    Sum v = acc[r];
 #pragma unroll
     for (int o = L / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     const int row = row0 + g * kAR + r;
-    if (l == 0 && live[r]) y[row] = v + (bias ? bias[row] : 0.0f);
+    if (l == 0 && live[r]) y[row] = (float)v + (bias ? bias[row] : 0.0f);
   }
 #endif
 }

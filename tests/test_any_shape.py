@@ -127,3 +127,24 @@ def test_any_shape_outlier(orc, dt, tokens, n, m):
     # each stays under 8 2^-24 of the result's norm (measured: about 4 2^-24)
     for t in range(tokens):
         assert orc.rel_l2(got[t], ref[t]) <= 8 * 2.0 ** -24, t
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,n,m,bound", [("q8_0", 8037, 288, 6.4e-8), ("q8_0", 8000, 32, 6e-8),
+                                          ("q4_0", 8000, 32, 9.5e-8), ("q4_0", 4096, 2880, 1.1e-7)])
+def test_any_length_gemv_error(orc, dt, n, m, bound):
+    """One token through the any-length GEMV is no further from 64 bits than the
+    fp32 dot products of the any-shape kernel (bounds: what those measured, and
+    sqrt(3.5) random roundings of 2.6e-8 for Q8_0, 4.9e-8, sqrt(8 to 14) for
+    Q4_0, 7.5e-8 to 9.7e-8)."""
+    import torch
+
+    from hypno_amd import _lib
+    print(f"{dt} n={n} m={m}", flush=True)
+    rng = np.random.default_rng(n + m)
+    w = (rng.standard_normal(n * m) * 0.02).astype(np.float32)
+    wb = orc.quantize_q4_0(w) if dt == "q4_0" else orc.quantize_q8_0(w)
+    x = rng.standard_normal((1, m)).astype(np.float32)
+    got = _run(_lib.load(), torch, dt, wb, x, np.zeros(n, np.float32), n, m, 1, 0)
+    f64 = orc.matmul_q4_0_f64 if dt == "q4_0" else orc.matmul_q8_0_f64
+    assert orc.rel_l2(got[0], f64(wb, x[0], None, n, m)) <= bound
