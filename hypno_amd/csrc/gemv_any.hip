@@ -191,6 +191,26 @@ gemv_any_kernel(float* __restrict__ y, const uint8_t* __restrict__ w, size_t w_b
 #pragma unroll
     for (int o = L / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     const int row = row0 + g * kAR + r;
+    // Integers times x leave fp32 where weights times x may not (|x| from 2^120
+    // on): a row that is not finite is computed again from the weights.
+    const bool again = live[r] && !(fabsf((float)v) < __builtin_inff());
+    if (__any(again)) {
+      float u = 0.0f;
+      if (again) {
+        for (int b = l; b < B; b += L) {
+          const uint8_t* blk = w + (size_t)row * row_bytes + (size_t)b * FT::kBytes;
+          const float d = f16_bits_to_f32((uint32_t)blk[0] | ((uint32_t)blk[1] << 8));
+          for (int i = 0; i < kBlockElems; i++) {
+            const int q = F == kFmtQ8_0 ? (int)blk[2 + i] - 128
+                                        : (int)((blk[2 + i / 2] >> (4 * (i & 1))) & 15) - 8;
+            u = fmaf((float)q * d, x[b * kBlockElems + i], u);
+          }
+        }
+      }
+#pragma unroll
+      for (int o = L / 2; o > 0; o >>= 1) u += __shfl_xor(u, o, 64);
+      if (again) v = u;
+    }
     if (l == 0 && live[r]) y[row] = (float)v + (bias ? bias[row] : 0.0f);
   }
 #endif

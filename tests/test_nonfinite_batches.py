@@ -1,4 +1,4 @@
-"""Batches that hold infinities, NaN or values near fp32's largest, on the GEMMs
+"""Tokens that hold infinities, NaN or values near fp32's largest, on the kernels
 for rows outside the tuned kernels' stages.  A token with one infinity has +-inf
 where that column's weight is not zero and NaN where it is, whatever finite
 values stand beside it; other tokens keep their fp32 accuracy."""
@@ -84,3 +84,26 @@ def test_f16_batch(orc, tokens, n, m):
         assert np.array_equal(got[:, r], one[:, r], equal_nan=True), r
     rest = np.setdiff1d(np.arange(n), list(inf))
     _check(orc, got[:, rest], x, w[rest].astype(np.float64))
+
+
+@pytest.mark.parametrize("dt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("n,m", [(33, 96), (300, 544), (257, 2080)])
+def test_one_token_near_the_largest(orc, dt, n, m):
+    """One token whose values times the blocks' integers leave fp32, times the
+    weights not."""
+    import torch
+    print(f"{dt} n={n} m={m}", flush=True)
+    rng = np.random.default_rng(n)
+    f = (rng.standard_normal(n * m) * 0.02).astype(np.float32)
+    wb = orc.quantize_q4_0(f) if dt == "q4_0" else orc.quantize_q8_0(f)
+    w = (orc.dequantize_q4_0 if dt == "q4_0" else orc.dequantize_q8_0)(wb)
+    w = w[:n * m].reshape(n, m).astype(np.float64)
+    x = rng.standard_normal((1, m)).astype(np.float32)
+    x[0, 3:40:3] = np.float32(3e38) * np.sign(x[0, 3:40:3])
+    got = _run(torch, f"hypno_hip_matmul_{dt}_dev", wb, x, n, m)
+    assert orc.normwise_err(got[0], x[0].astype(np.float64) @ w.T) <= 2e-5
+    x[0, 3] = np.inf
+    got = _run(torch, f"hypno_hip_matmul_{dt}_dev", wb, x, n, m)
+    with np.errstate(invalid="ignore"):
+        want = w[:, 3] * np.inf
+    assert np.array_equal(got[0], want.astype(np.float32), equal_nan=True)
