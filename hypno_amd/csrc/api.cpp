@@ -450,17 +450,16 @@ int q4_0_col_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const
   hipError_t e;
   // Several tokens: the pair GEMM, against the one-token kernel over groups of
   // tokens.  Measured per call (us, one-token kernel and GEMM): 2048 x 2048
-  // 16 / 17.2 at 8, 26.4 / 17.5 at 16, 144 / 20.5 at 128; 5632 x 2048 31 / 17.5
-  // at 8, 52 / 17 at 16, 412 / 28 at 128; 14336 x 4096 52 / 28 at 8, 2885 / 174
-  // at 512; 1024 x 512 14.7 / 17 at 16, 19.4 / 17 at 64: about
-  // 8 us and 0.25 us per million weights and token (0.11 beyond 32M, which
-  // fill the chip) against 17 us (three launches), 0.17 us per million weights
-  // and 0.006 per million and token.  Fewer than 8 tokens stay with the
+  // 26 / 14.5 at 16; 5632 x 2048 31 / 20 at 8, 391 / 35 at 128; 14336 x 4096 53 /
+  // 37 at 8, 2915 / 340 at 512; 544 x 4160 30 / 20 at 18; 640 x 704 28 / 14 at 91:
+  // about 8 us and 0.25 us per million weights and token (0.11 beyond 32M, which
+  // fill the chip) against 17 us (three launches), 0.25 us per million weights
+  // and 0.0105 per million and token.  Fewer than 8 tokens stay with the
   // one-token kernel, whose rows equal one-token calls bit for bit.
   {
     const double mw = (double)n * m * 1e-6;
     const double one = 8.0 + batch * mw * (mw < 32.0 ? 0.25 : 0.11);
-    const double many = 17.0 + mw * (0.17 + 0.006 * batch);
+    const double many = 17.0 + mw * (0.25 + 0.0105 * batch);
     if (batch >= 8 && many < one && q4_0_col_gemm_ok(w, w_len, n, m, batch)) {
       const size_t bytes = q4_0_col_gemm_workspace_bytes(n, m, batch, cus);
       if (workspace_can_hold(ds, s, bytes)) {
@@ -533,10 +532,10 @@ int f16_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const floa
     return HYPNO_HIP_OK;
   }
   // Rows that are no multiple of the GEMMs' 64-column stages: the fp32-accurate
-  // pair GEMM, against one GEMV per token (us: 2880 x 7200 24.2 / 26.3 at 2
-  // tokens, 29.3 / 823 at 64; 4096 x 2080 12.7 / 12.6 at 2, 12.9 / 48.5 at 8;
-  // 1024 x 544 11.0 / 6.1 at 2, 12.9 / 23.4 at 8).
-  if (batch >= 2 && (batch >= 4 || (double)n * m * batch >= 17e6) &&
+  // pair GEMM, against one GEMV per token (us: 2880 x 7200 23.1 / 34.2 at 3
+  // tokens, 33 / 800 at 64; 4096 x 2080 13.4 / 15.9 at 3, 13.8 / 21.3 at 4; 1024 x
+  // 544 11.3 / 10.2 at 3, 11.5 / 12.7 at 4; two tokens 13.5 / 10.1 and 22.9 / 22.8).
+  if (batch >= 3 && (batch >= 4 || (double)n * m * batch >= 17e6) &&
       f16_pair_gemm_ok(w, n, m, batch)) {
     const size_t bytes = f16_pair_gemm_workspace_bytes(n, m, batch, cus);
     if (workspace_can_hold(ds, s, bytes)) {

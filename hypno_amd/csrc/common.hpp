@@ -411,16 +411,11 @@ hipError_t launch_block_gemm_f16x(const BlockPlan& p, int fmt, float* y, const u
 size_t x_split_bytes(size_t batch, size_t m);
 int* x_split_exponents(void* xs, size_t batch, size_t m);
 hipError_t launch_x_split(void* xs, const float* x, size_t batch, size_t m, hipStream_t s);
-// X fp32 [batch][m] -> fp16 [batch][kp] hi parts and a plane of lo parts in
-// natural column order, per-row exponents at xexp; with `clear`, *clear = 0
-// and the exponent of a row holding inf or NaN is INT_MIN.
-hipError_t launch_x_hilo(void* xh, int* xexp, const float* x, size_t batch, size_t m, size_t kp,
-                         uint32_t* clear, hipStream_t s);
 // y[mn] = the sum of `splits` planes of mn floats in order (+ bias[i % n]).
 hipError_t launch_split_reduce(float* y, const float* part, const float* bias, size_t mn, size_t n,
                                int splits, hipStream_t s);
 
-// fp32-accurate batched GEMMs on fp16 operand pairs (gemm_pair.hip):
+// fp32-accurate batched GEMMs on bf16 operand parts (gemm_pair.hip):
 // column-major Q4_0, and fp16 weights with any m % 32 == 0.
 bool q4_0_col_gemm_ok(const uint8_t* w, size_t w_len, size_t n, size_t m, size_t batch);
 size_t q4_0_col_gemm_workspace_bytes(size_t n, size_t m, size_t batch, int num_cus);

@@ -480,15 +480,23 @@ __global__ void __launch_bounds__(kBThreads, 1) gemm_block_kernel(const BlockArg
 #endif
 }
 
-// Y = the planes in split order (+ bias).
+// Y = the planes (+ bias): plane z in sum z % 4, the four then added, an order of
+// its own that is the same on every run (up to 64 planes as one chain rounded
+// more than the fp32 dot products: 16 tokens, column-major 2048 x 2048 in 32
+// pieces 1.16e-7 against 1.15e-7).
 __global__ void __launch_bounds__(256)
 block_split_reduce_kernel(float* __restrict__ y, const float* __restrict__ part,
                           const float* __restrict__ bias, size_t mn, int n, int splits) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= mn) return;
-  float v = part[i];
-  for (int z = 1; z < splits; z++) v += part[(size_t)z * mn + i];
-  y[i] = v + (bias ? bias[i % n] : 0.0f);
+  float v[4] = {part[i], 0.0f, 0.0f, 0.0f};
+  for (int z = 1; z < 4 && z < splits; z++) v[z] = part[(size_t)z * mn + i];
+  for (int z = 4; z < splits; z += 4) {
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (z + k < splits) v[k] += part[(size_t)(z + k) * mn + i];
+  }
+  y[i] = ((v[0] + v[1]) + (v[2] + v[3])) + (bias ? bias[i % n] : 0.0f);
 }
 
 // X fp32 [M][K] -> three bf16 planes [M][Kp], `plane` vectors apart, one
@@ -592,107 +600,6 @@ x_rows_split_kernel(u32x4* __restrict__ xh, int* __restrict__ xexp, const float*
   if (t == 0) xexp[row] = -sh;
 }
 
-// X fp32 [M][K] -> fp16 [M][Kp] hi parts and, `plane` vectors on, lo parts,
-// one work-group of 256 threads per row: scaled by 2^sh (sh puts the row's
-// largest |x| in [2^14, 2^15); 0 for an all-zero row or one holding inf or
-// NaN), xexp[row] = -sh, columns K .. Kp - 1 zero.  The row is
-// read once if it fits the registers (K <= 16384 and 16-byte aligned), twice
-// otherwise.  With `clear`, *clear is set to 0 and the exponent of a row
-// holding inf or NaN to INT_MIN.
-__global__ void __launch_bounds__(256)
-x_rows_block_kernel(u32x4* __restrict__ xh, int* __restrict__ xexp, const float* __restrict__ x,
-                    size_t plane, int K, int Kp, uint32_t* __restrict__ clear) {
-  __shared__ uint32_t red[4];
-  const int row = blockIdx.x;
-  const int t = threadIdx.x;
-  if (clear && row == 0 && t == 0) *clear = 0;
-  const int groups = K / 8, gp = Kp / 8;
-  u32x4* dst = xh + (size_t)row * gp;
-  const float* src = x + (size_t)row * K;
-  const bool al = ((uintptr_t)src & 15) == 0;
-  const bool keep = al && groups <= 256 * kXG;
-  float4 v[kXG][2];
-  uint32_t mb = 0;  // largest |x| by bit pattern (inf and NaN above every finite value)
-  auto load8 = [&](int g, float4& lo, float4& hi) {
-    const float* p = src + (size_t)g * 8;
-    if (al) {
-      lo = load_global<float4>(p);
-      hi = load_global<float4>(p + 4);
-    } else {
-      lo = make_float4(p[0], p[1], p[2], p[3]);
-      hi = make_float4(p[4], p[5], p[6], p[7]);
-    }
-  };
-  auto amax8 = [&](const float4& lo, const float4& hi) {
-    const float e[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-#pragma unroll
-    for (int i = 0; i < 8; i++) mb = max(mb, __float_as_uint(e[i]) & 0x7FFFFFFFu);
-  };
-  if (keep) {
-#pragma unroll
-    for (int u = 0; u < kXG; u++)
-      if (t + 256 * u < groups) load8(t + 256 * u, v[u][0], v[u][1]);
-#pragma unroll
-    for (int u = 0; u < kXG; u++)
-      if (t + 256 * u < groups) amax8(v[u][0], v[u][1]);
-  } else {
-    for (int g = t; g < groups; g += 256) {
-      float4 lo, hi;
-      load8(g, lo, hi);
-      amax8(lo, hi);
-    }
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, off, 64));
-  if ((t & 63) == 0) red[t >> 6] = mb;
-  __syncthreads();
-  mb = max(max(red[0], red[1]), max(red[2], red[3]));
-  const float amax = __uint_as_float(mb);
-  int sh = 0;
-  if (amax > 0.0f && amax < __builtin_inff()) sh = 15 - __builtin_amdgcn_frexp_expf(amax);
-  auto put = [&](int g, const float4& lo, const float4& hi) {
-    const float e[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-    u32x4 a, b;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      // (a finite value past fp16's range, which only a row without a scale of
-      // its own can hold, stays finite: that row's outputs are the infinity's)
-      auto in_range = [](float f) {
-        return fabsf(f) < __builtin_inff() ? fminf(fmaxf(f, -65504.0f), 65504.0f) : f;
-      };
-      const float s0 = in_range(ldexpf(e[2 * j], sh));
-      const float s1 = in_range(ldexpf(e[2 * j + 1], sh));
-      const _Float16 h0 = (_Float16)s0, h1 = (_Float16)s1;
-      a[j] = (uint32_t)__builtin_bit_cast(uint16_t, h0) |
-             ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-      // (inf - inf: the hi part alone carries an infinity)
-      const float r0 = s0 - (float)h0, r1 = s1 - (float)h1;
-      const _Float16 l0 = (_Float16)(r0 == r0 ? r0 : 0.0f);
-      const _Float16 l1 = (_Float16)(r1 == r1 ? r1 : 0.0f);
-      b[j] = (uint32_t)__builtin_bit_cast(uint16_t, l0) |
-             ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
-    }
-    dst[g] = a;
-    dst[plane + g] = b;
-  };
-  if (keep) {
-#pragma unroll
-    for (int u = 0; u < kXG; u++)
-      if (t + 256 * u < groups) put(t + 256 * u, v[u][0], v[u][1]);
-  } else {
-    for (int g = t; g < groups; g += 256) {
-      float4 lo, hi;
-      load8(g, lo, hi);
-      put(g, lo, hi);
-    }
-  }
-  if (t < gp - groups) {
-    dst[groups + t] = u32x4{0u, 0u, 0u, 0u};
-    dst[plane + groups + t] = u32x4{0u, 0u, 0u, 0u};
-  }
-  if (t == 0) xexp[row] = clear && mb >= 0x7F800000u ? (int)0x80000000u : -sh;
-}
-
 size_t rup(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 }  // namespace
@@ -700,9 +607,9 @@ size_t rup(size_t v, size_t a) { return (v + a - 1) / a * a; }
 // Geometry chosen for a shape: 32-row tiles per wave and K pieces.
 //
 // Costs (microseconds, fitted to 26 shapes at every number of pieces; the plans
-// they choose measured 1.3% above the best on average): a 64-K stage
-// 0.85 / 1.2 on 32- / 64-row tiles, a round of work-groups (one per CU) ~3
-// more to fill and drain; K pieces add the reduction launch (~2.5) and the
+// they choose measured 0.2% above the best on average, 1% at most): a 64-K stage
+// 0.95 / 1.2 on 32- / 64-row tiles, a round of work-groups (one per CU) ~3 more
+// to fill and drain; K pieces add the reduction launch (~2.5), 0.3 each and the
 // partial planes' traffic (~2 TB/s a way).
 BlockPlan block_plan(size_t n, size_t m, size_t batch, int num_cus) {
   const size_t tn = (n + kBN - 1) / kBN;
@@ -713,12 +620,12 @@ BlockPlan block_plan(size_t n, size_t m, size_t batch, int num_cus) {
     if (mt > 1 && (size_t)16 * mt >= batch) break;  // taller tiles than the rows
     const size_t tm = (batch + 32 * mt - 1) / (32 * mt);
     const size_t tiles = tm * tn;
-    const double stage_us = mt == 2 ? 1.2 : 0.85;
+    const double stage_us = mt == 2 ? 1.2 : 0.95;
     for (size_t sp = 1; sp <= std::min<size_t>(steps, 64); sp++) {
       const size_t wgs = tiles * sp;
       const size_t rounds = (wgs + num_cus - 1) / num_cus;
       double cost = (double)rounds * ((double)((steps + sp - 1) / sp) * stage_us + 3.0);
-      if (sp > 1) cost += 2.5 + (double)sp * (double)(batch * n * 4) / 2.0e6;
+      if (sp > 1) cost += 2.5 + (double)sp * (0.3 + (double)(batch * n * 4) / 2.0e6);
       if (cost < best_cost * 0.999) {
         best_cost = cost;
         best = BlockPlan{mt, (int)sp, cost};
@@ -885,13 +792,6 @@ hipError_t launch_split_reduce(float* y, const float* part, const float* bias, s
                                int splits, hipStream_t s) {
   hipLaunchKernelGGL(block_split_reduce_kernel, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0,
                      s, y, part, bias, mn, (int)n, splits);
-  return hipGetLastError();
-}
-
-hipError_t launch_x_hilo(void* xh, int* xexp, const float* x, size_t batch, size_t m, size_t kp,
-                         uint32_t* clear, hipStream_t s) {
-  hipLaunchKernelGGL(x_rows_block_kernel, dim3((unsigned)batch), dim3(256), 0, s,
-                     static_cast<u32x4*>(xh), xexp, x, batch * kp / 8, (int)m, (int)kp, clear);
   return hipGetLastError();
 }
 

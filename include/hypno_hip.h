@@ -48,15 +48,19 @@
  *         lo (x 2^s = hi + lo to ~2^-22), on MFMA against the fp16 weights
  *         with fp32 accumulation (the 1e-4 bar per token; fp32 FMAs token by
  *         token if x is not 16-byte aligned); M >= 16 as the Q4_0 GEMM with
- *         fp16 weights.  Rows of m % 64 == 32: hi and lo rows at every M.
+ *         fp16 weights.  Rows of m % 64 == 32: from 3 tokens (3 from
+ *         17M products on) activations in three bf16 parts and weights in two,
+ *         both exact, on MFMA with fp32 accumulation; fewer fp32 FMAs token
+ *         by token.
  *       Q8_0: M < 16 each token's activations as three exact int8 digit
  *         planes per block (to 2^-23), each weight block read once for 2 to 8
  *         tokens; M >= 16 as the Q4_0 GEMM with exact integer weights, or
  *         where that is faster weights expanded once to fp16
  *         (row-normalised, relative 2^-11) and the FP16 GEMM.
  *       Column-major Q4_0: fp32 FMAs token by token; from 8 tokens, where it
- *         is faster, exact fp16 pairs of weights times hi/lo pairs of
- *         activations on MFMA (the same 1e-4 bar per token).
+ *         is faster, weights in two bf16 parts times activations in three,
+ *         both exact, on MFMA with fp32 accumulation (the same 1e-4 bar per
+ *         token).
  *   - Every function returns a status (HYPNO_HIP_OK on success) and never
  *     aborts the process.  hypno_hip_last_error() describes the last failure
  *     on the calling thread.

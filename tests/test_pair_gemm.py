@@ -1,4 +1,4 @@
-"""Batches on the fp16-pair GEMM: column-major Q4_0 at many tokens and fp16
+"""Batches on the pair GEMM: column-major Q4_0 at many tokens and fp16
 weights whose rows are no multiple of 64, at the edges of its tiles (row tiles
 of 32, 64 and 128 tokens, 256 output columns, 64-column stages cut in half),
 with short buffers, scales past fp16's products, infinities and biases."""
@@ -45,7 +45,7 @@ def test_col_major_many_tokens(orc, tokens, n, m, cut):
     bias = rng.standard_normal(n).astype(np.float32)
     got = _col(torch, wb, x, bias, n, m)
     ref = _col_f64(orc, wb, x, bias, n, m)
-    # fp32 sums and pairs exact to 2^-22: random error well under sqrt(K) 2^-22
+    # fp32 sums of exact products: random error well under sqrt(K) 2^-24
     for t in range(tokens):
         assert orc.normwise_err(got[t], ref[t]) <= 2e-5, t
 
@@ -110,3 +110,55 @@ def test_f16_half_stage_rows(orc, tokens, n, m):
     ref = x.astype(np.float64) @ w.reshape(n, m).astype(np.float64).T
     for t in range(tokens):
         assert orc.normwise_err(got[t], ref[t]) <= 2e-5, t
+
+
+def _outliers(rng, tokens, m, k):
+    """Ordinary tokens, and the same with values 2^12 to 2^100 at column k."""
+    x = rng.standard_normal((tokens, m)).astype(np.float32)
+    big = x.copy()
+    big[:, k] = np.ldexp(np.float32(1.0), 12 + np.arange(tokens) * 88 // (tokens - 1))
+    x[:, k] = 0.0
+    return x, big
+
+
+# Exact products; the random rounding of their fp32 sums stays under 4 2^-24 of
+# the result's norm (measured: 1 to 2 2^-24).
+OUTLIER_TOL = 4 * 2.0 ** -24
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,n,m", [(128, 5632, 2048), (16, 2048, 2080)])
+def test_col_major_outlier(orc, tokens, n, m):
+    """Tokens whose largest value meets weights of zero: outputs are as accurate
+    as if that input were not there."""
+    import torch
+    print(f"col tokens={tokens} n={n} m={m}", flush=True)
+    rng = np.random.default_rng(n)
+    w = (rng.standard_normal((m, n)) * 0.02).astype(np.float32)
+    w[100] = 0.0
+    wb = orc.quantize_q4_0(w.ravel())
+    x, big = _outliers(rng, tokens, m, 100)
+    got = _col(torch, wb, big, None, n, m)
+    ref = _col_f64(orc, wb, x, None, n, m)
+    for t in range(tokens):
+        assert orc.rel_l2(got[t], ref[t]) <= OUTLIER_TOL, t
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,n,m", [(200, 7200, 2848), (8, 4096, 2080)])
+def test_f16_outlier(orc, tokens, n, m):
+    import torch
+
+    import hypno_amd as hk
+    print(f"f16 tokens={tokens} n={n} m={m}", flush=True)
+    rng = np.random.default_rng(n)
+    w = (rng.standard_normal((n, m)) * 0.02).astype(np.float16)
+    w[:, 100] = 0.0
+    x, big = _outliers(rng, tokens, m, 100)
+    y = torch.full((tokens, n), float("nan"), device="cuda")
+    hk.batch_matmul(y, torch.from_numpy(w.view(np.uint8)).cuda(), hk.DType.FP16,
+                    torch.from_numpy(big).cuda(), n, m, tokens)
+    torch.cuda.synchronize()
+    got, ref = y.cpu().numpy(), x.astype(np.float64) @ w.astype(np.float64).T
+    for t in range(tokens):
+        assert orc.rel_l2(got[t], ref[t]) <= OUTLIER_TOL, t
