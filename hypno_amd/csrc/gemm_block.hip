@@ -637,20 +637,23 @@ BlockPlan block_plan(size_t n, size_t m, size_t batch, int num_cus) {
 }
 
 // The same for x rounded once to fp16 (m % 64 == 0), with no more than
-// `planes` bytes of partial planes.  A stage costs 0.95 / 1.25 / 2.3 on 64- /
-// 128- / 256-row tiles (Q8_0, twice the weight bytes: 1.0 / 1.42 / 2.35); K
-// pieces write planes that the reduction reads, ~3 TB/s in all.
+// `planes` bytes of partial planes.  A stage costs 1.0 / 1.42 / 2.35 on 64- /
+// 128- / 256-row tiles of Q8_0; K pieces write planes that the reduction reads,
+// ~3 TB/s in all.  Q4_0 has the 256-row tiles only (2.3): on lower ones the
+// 16x16x32 kernel is as fast or faster (512 x 14336, K 4096: 90 us against 91;
+// 2048 x 4096, K 4096: 98 / 100; 1024 x 4096, K 14336: 173 / 179; 400 x 14336, K
+// 2048: 49.5 / 50.7).
 BlockPlan block_plan_f16x(int fmt, size_t n, size_t m, size_t batch, int num_cus, size_t planes) {
   const size_t tn = (n + kBN - 1) / kBN;
   const size_t steps = m / kBStageK;
-  BlockPlan best{2, 1, 1e300};
+  const bool q8 = fmt == kFmtQ8_0;
+  BlockPlan best{q8 ? 2 : 8, 1, 1e300};
   for (int mt : {2, 4, 8}) {
+    if (!q8 && mt != 8) continue;
     if (mt > 2 && (size_t)16 * mt >= batch) break;  // taller tiles than the rows
     const size_t tm = (batch + 32 * mt - 1) / (32 * mt);
     const size_t tiles = tm * tn;
-    const bool q8 = fmt == kFmtQ8_0;
-    const double stage_us = mt == 8 ? (q8 ? 2.35 : 2.3) : mt == 4 ? (q8 ? 1.42 : 1.25)
-                                                                  : (q8 ? 1.0 : 0.95);
+    const double stage_us = mt == 8 ? (q8 ? 2.35 : 2.3) : mt == 4 ? 1.42 : 1.0;
     for (size_t sp = 1; sp <= std::min<size_t>(steps, 64); sp++) {
       if (sp > 1 && sp * batch * n * 4 > planes) break;
       const size_t rounds = (tiles * sp + num_cus - 1) / num_cus;
@@ -756,8 +759,13 @@ static hipError_t launch_block_single(const BlockPlan& p, const BlockArgs& a, hi
     return hipGetLastError();
   };
   if (p.mt == 8) return go(gemm_block_kernel<FMT, 8, false, 1>, BlockGeom<FMT, 8, false, 1>::kLds);
-  if (p.mt == 4) return go(gemm_block_kernel<FMT, 4, false, 1>, BlockGeom<FMT, 4, false, 1>::kLds);
-  return go(gemm_block_kernel<FMT, 2, false, 1>, BlockGeom<FMT, 2, false, 1>::kLds);
+  if constexpr (FMT == kFmtQ8_0) {
+    if (p.mt == 4)
+      return go(gemm_block_kernel<FMT, 4, false, 1>, BlockGeom<FMT, 4, false, 1>::kLds);
+    if (p.mt == 2)
+      return go(gemm_block_kernel<FMT, 2, false, 1>, BlockGeom<FMT, 2, false, 1>::kLds);
+  }
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_block_gemm_f16x(const BlockPlan& p, int fmt, float* y, const uint8_t* w,

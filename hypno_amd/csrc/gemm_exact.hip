@@ -542,11 +542,13 @@ size_t planes_bytes(int splits, size_t batch, size_t n) {
 // Whether the block GEMM on the same fp16 rows (32x32x16 MFMAs, 256 columns a
 // work-group) is the faster of the two: its 256 x 256 tiles spend half the
 // stages and LDS reads of this kernel's 256 x 128 ones per product, where a
-// grid of them comes out even.  The factor is what this kernel's tall tiles
-// measured above the model on a full chip (3 to 8%).  Per call, this kernel
-// and the other (us): 2048 x 14336, K 4096: 375 / 296; 1024 x 14336, K 4096:
-// 210 / 155; 2048 x 5632, K 2048: 96 / 83; left here: 512 x 8192, K 3072:
-// 53.5 / 55.0; 512 x 3072, K 8192: 54.2 / 55.7; 2048 x 2048, K 5632: 85 / 87.
+// grid of them comes out even.  The models put this kernel up to 3% low and
+// those tiles 4% high on a full chip: the measured times cross where the
+// modelled ones are at 1.07 to 1.09 of each other.  Per call, this kernel and the
+// other (us): 2048 x 14336, K 4096: 332 / 290; 1024 x 14336, K 4096: 165 / 145;
+// 2048 x 5632, K 2048: 92 / 81; 557 x 15360, K 4416 (modelled at 1.03 of this
+// one): 156 / 144; left here: 1291 x 7040, K 6848 (1.10): 228 / 220; 1841 x 17088, K
+// 1600 (1.08): 183 / 190; 512 x 14336, K 4096: 90 / 136.
 bool use_block(const ExactPlan& p, const BlockPlan& b) { return b.cost < 1.05 * p.cost; }
 
 }  // namespace

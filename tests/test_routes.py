@@ -1,0 +1,72 @@
+"""Which kernels a call runs, and what it allocates, on a HIP runtime that runs
+nothing (fake_hip/): the rules of the dispatch on the CPU."""
+import json
+import os
+import re
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def calls(tmp_path_factory):
+    from hypno_amd import _lib
+    so = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", so,
+                    os.path.join(HERE, "fake_hip", "fake_hip.cpp")], check=True)
+
+    def run(*steps):
+        p = subprocess.run([sys.executable, os.path.join(HERE, "fake_hip", "calls.py"), so,
+                            _lib.LIB_PATH, json.dumps(steps)], capture_output=True, text=True,
+                           timeout=100)
+        assert p.returncode == 0, p.stderr
+        return json.loads(p.stdout)
+
+    return run
+
+
+def _kernels(result):
+    """Short names of a call's launches: mangled name -> identifier<int and bool
+    template arguments>."""
+    st, log = result
+    assert st == 0, result
+    out = []
+    for line in log:
+        if line.startswith("launch "):
+            name = line.split()[1]
+            # the last length-prefixed identifier before the template arguments
+            ident = args = ""
+            i = name.index("5hypno") + 6
+            while i < len(name):
+                if name.startswith("12_GLOBAL__N_1", i):
+                    i += 14
+                    continue
+                g = re.match(r"(\d+)", name[i:])
+                if not g:
+                    break
+                k = i + len(g.group(1))
+                ident, i = name[k:k + int(g.group(1))], k + int(g.group(1))
+            if name[i:i + 1] == "I":
+                args = re.match(r"I((?:L[ib]\d+E)+)", name[i:])
+                args = ",".join(re.findall(r"L[ib](\d+)E", args.group(1))) if args else ""
+            out.append(f"{ident}<{args}>" if args else ident)
+    return out
+
+
+# Q4_0 prompts: 256 x 256 block tiles where they fill the chip evenly, the 16x16x32
+# kernel elsewhere (us, that kernel and block tiles of 128 / 256 rows: 512 x 14336,
+# K 4096 90 / 91 / 136; 2048 x 4096, K 4096 98 / 100 / 141; 2048 x 4096, K 14336
+# 326 / 323 / 458; 1024 x 14336, K 4096 165 / 168 / 145; 2048 x 14336 332 / 340 / 290).
+@pytest.mark.parametrize("tokens,n,m,block", [
+    (512, 14336, 4096, False), (2048, 4096, 4096, False), (2048, 4096, 14336, False),
+    (2048, 3072, 8192, False), (1024, 4096, 14336, False), (512, 8192, 3072, False),
+    (512, 3072, 8192, False), (1500, 11008, 4096, False), (3000, 5632, 2048, False),
+    (2048, 14336, 4096, True), (1024, 14336, 4096, True), (2048, 5632, 2048, True),
+    (2048, 8192, 3072, True), (4096, 4096, 14336, True), (2048, 6144, 4096, True)])
+def test_q4_0_prompt_tiles(calls, tokens, n, m, block):
+    got = _kernels(calls(["q4_0", n, m, tokens])[0])
+    assert ("gemm_block_kernel<0,8,0,1>" in got) == block, got
+    assert any(k.startswith("q4_0_gemm_exact_kernel") for k in got) == (not block), got
