@@ -66,6 +66,7 @@ hipError_t ensure(DevBuf& b, size_t bytes, hipStream_t sync) {
   const size_t want = bytes < 256 ? 256 : bytes;
   hipError_t e = hipMalloc(&b.p, want);
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // (returned here, not for the next launch to report)
     b.p = nullptr;
     return e;
   }
@@ -89,6 +90,7 @@ hipError_t ensure_host(DevBuf& b, size_t bytes, hipStream_t sync) {
   const size_t want = (bytes < 65536 ? 65536 : bytes + 4095) / 4096 * 4096;
   hipError_t e = hipHostMalloc(&b.p, want, hipHostMallocMapped);
   if (e != hipSuccess) {
+    (void)hipGetLastError();
     b.p = nullptr;
     return e;
   }
@@ -170,9 +172,18 @@ struct WsLock {
   void* p = nullptr;
 };
 
-// Locks stream s's workspace on the device of `ds` and grows it to `bytes`.
-int lock_workspace(DeviceState* ds, hipStream_t s, size_t bytes, WsLock& out,
-                   const char* what) {
+// Whether stream s is under graph capture (where nothing can be allocated).
+bool is_capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();  // (the NULL stream while another is: not for the next launch to report)
+  return true;
+}
+
+// Locks stream s's workspace on the device of `ds` and grows it to `bytes`;
+// `optional`: not if s is under capture.
+hipError_t grow_workspace(DeviceState* ds, hipStream_t s, size_t bytes, WsLock& out,
+                          bool optional) {
   StreamWs* w = nullptr;
   {
     std::lock_guard<std::mutex> g(g_mu);
@@ -181,28 +192,26 @@ int lock_workspace(DeviceState* ds, hipStream_t s, size_t bytes, WsLock& out,
     w = slot.get();
   }
   out.lk = std::unique_lock<std::mutex>(w->mu);
+  if (optional && !(w->buf.p && w->buf.cap >= bytes) && is_capturing(s))
+    return hipErrorStreamCaptureUnsupported;
   hipError_t e = ensure(w->buf, bytes, s);
-  if (e != hipSuccess) return hip_fail(e, what);
+  if (e != hipSuccess) return e;
   out.p = w->buf.p;
-  return HYPNO_HIP_OK;
+  return hipSuccess;
 }
 
-// Whether stream s's workspace holds `bytes`, or may grow to: a stream under
-// graph capture cannot allocate, so there a call whose plain kernels need no
-// workspace takes those instead.
-bool workspace_can_hold(DeviceState* ds, hipStream_t s, size_t bytes) {
-  StreamWs* w = nullptr;
-  {
-    std::lock_guard<std::mutex> g(g_mu);
-    auto it = ds->workspaces.find(s);
-    if (it != ds->workspaces.end()) w = it->second.get();
-  }
-  if (w) {
-    std::lock_guard<std::mutex> g(w->mu);
-    if (w->buf.p && w->buf.cap >= bytes) return true;
-  }
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+int lock_workspace(DeviceState* ds, hipStream_t s, size_t bytes, WsLock& out, const char* what) {
+  hipError_t e = grow_workspace(ds, s, bytes, out, false);
+  return e == hipSuccess ? HYPNO_HIP_OK : hip_fail(e, what);
+}
+
+// The same for a call that has other kernels to run: false where the workspace
+// does not hold `bytes` and cannot grow (device memory is full, or the stream is
+// under capture).
+bool try_workspace(DeviceState* ds, hipStream_t s, size_t bytes, WsLock& out) {
+  if (grow_workspace(ds, s, bytes, out, true) == hipSuccess) return true;
+  out.lk.unlock();
+  return false;
 }
 
 // [a, a + na) and [b, b + nb) share a byte (empty ranges share none).
@@ -251,13 +260,12 @@ int try_block_gemm(int fmt, float* y, const uint8_t* w, size_t w_len, const floa
     return HYPNO_HIP_OK;
   const BlockPlan p = block_plan(n, m, batch, cus);
   const size_t bytes = block_gemm_workspace_bytes(p, n, m, batch);
-  if (fixed ? bytes > fixed->bytes : !workspace_can_hold(ds, s, bytes)) return HYPNO_HIP_OK;
   WsLock ws;
   if (fixed) {
+    if (bytes > fixed->bytes) return HYPNO_HIP_OK;
     ws.p = fixed->ptr;
-  } else {
-    int st = lock_workspace(ds, s, bytes, ws, "block GEMM workspace");
-    if (st) return st;
+  } else if (!try_workspace(ds, s, bytes, ws)) {
+    return HYPNO_HIP_OK;
   }
   hipError_t e = launch_block_gemm(p, fmt, y, w, x, bias, n, m, batch, ws.p, s);
   if (e != hipSuccess) return hip_fail(e, "block GEMM launch");
@@ -323,11 +331,18 @@ int q4_0_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const flo
   // numerics modes are one)
   if (batch >= kGemmMinBatch && (!gemm_folded() || m % 256 != 0) &&
       q4_0_gemm_exact_ok(w, w_len, n, m, batch)) {
+    // (the tile kernel below, which also takes K % 256 != 0, needs no more than
+    // the fp16 rows)
     const size_t bytes = q4_0_gemm_exact_workspace_bytes(batch, n, m, cus);
-    if (m % 256 == 0 || !fixed || bytes <= fixed->bytes) {
-      WsLock ws;
+    WsLock ws;
+    bool have = true;
+    if (m % 256 == 0 || (fixed && bytes <= fixed->bytes)) {
       st = scratch_for(bytes, ws, "GEMM workspace");
       if (st) return st;
+    } else {
+      have = !fixed && try_workspace(ds, s, bytes, ws);
+    }
+    if (have) {
       e = launch_q4_0_gemm_exact(y, w, x, bias, n, m, batch, ws.p, cus, s);
       if (e != hipSuccess) return hip_fail(e, "q4_0 exact GEMM launch");
       return HYPNO_HIP_OK;
@@ -390,11 +405,15 @@ int q8_0_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const flo
   }
   hipError_t e;
   if (batch >= kGemmMinBatch && q8_0_gemm_ok(n, m, batch)) {
+    const size_t block = q8_0_gemm_workspace_bytes(w, batch, n, m, cus, false);
     WsLock ws;
-    st = lock_workspace(ds, s, q8_0_gemm_workspace_bytes(w, batch, n, m, cus), ws,
-                        "Q8_0 GEMM workspace");
-    if (st) return st;
-    e = launch_q8_0_gemm(y, w, x, bias, n, m, batch, ws.p, cus, s);
+    const bool expand = !block || !try_workspace(ds, s, block, ws);
+    if (expand) {
+      st = lock_workspace(ds, s, q8_0_gemm_workspace_bytes(w, batch, n, m, cus, true), ws,
+                          "Q8_0 GEMM workspace");
+      if (st) return st;
+    }
+    e = launch_q8_0_gemm(y, w, x, bias, n, m, batch, ws.p, cus, expand, s);
     if (e != hipSuccess) return hip_fail(e, "q8_0 GEMM launch");
     return HYPNO_HIP_OK;
   }
@@ -461,11 +480,8 @@ int q4_0_col_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const
     const double one = 8.0 + batch * mw * (mw < 32.0 ? 0.25 : 0.11);
     const double many = 17.0 + mw * (0.25 + 0.0105 * batch);
     if (batch >= 8 && many < one && q4_0_col_gemm_ok(w, w_len, n, m, batch)) {
-      const size_t bytes = q4_0_col_gemm_workspace_bytes(n, m, batch, cus);
-      if (workspace_can_hold(ds, s, bytes)) {
-        WsLock ws;
-        st = lock_workspace(ds, s, bytes, ws, "column-major workspace");
-        if (st) return st;
+      WsLock ws;
+      if (try_workspace(ds, s, q4_0_col_gemm_workspace_bytes(n, m, batch, cus), ws)) {
         e = launch_q4_0_col_gemm(y, w, w_len, x, bias, n, m, batch, ws.p, cus, s);
         if (e != hipSuccess) return hip_fail(e, "column-major GEMM launch");
         return HYPNO_HIP_OK;
@@ -537,11 +553,8 @@ int f16_dev(float* y, const uint8_t* w, size_t w_len, const float* x, const floa
   // 544 11.3 / 10.2 at 3, 11.5 / 12.7 at 4; two tokens 13.5 / 10.1 and 22.9 / 22.8).
   if (batch >= 3 && (batch >= 4 || (double)n * m * batch >= 17e6) &&
       f16_pair_gemm_ok(w, n, m, batch)) {
-    const size_t bytes = f16_pair_gemm_workspace_bytes(n, m, batch, cus);
-    if (workspace_can_hold(ds, s, bytes)) {
-      WsLock ws;
-      st = lock_workspace(ds, s, bytes, ws, "GEMM workspace");
-      if (st) return st;
+    WsLock ws;
+    if (try_workspace(ds, s, f16_pair_gemm_workspace_bytes(n, m, batch, cus), ws)) {
       e = launch_f16_pair_gemm(y, w, x, bias, n, m, batch, ws.p, cus, s);
       if (e != hipSuccess) return hip_fail(e, "f16 pair GEMM launch");
       return HYPNO_HIP_OK;

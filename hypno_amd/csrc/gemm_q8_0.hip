@@ -113,23 +113,25 @@ static BlockPlan q8_0_plan(const uint8_t* w, size_t n, size_t m, size_t batch, i
   return b;
 }
 
-size_t q8_0_gemm_workspace_bytes(const uint8_t* w, size_t batch, size_t n, size_t m,
-                                 int num_cus) {
-  const BlockPlan b = q8_0_plan(w, n, m, batch, num_cus);
-  if (b.splits)
+size_t q8_0_gemm_workspace_bytes(const uint8_t* w, size_t batch, size_t n, size_t m, int num_cus,
+                                 bool expand) {
+  if (!expand) {
+    const BlockPlan b = q8_0_plan(w, n, m, batch, num_cus);
+    if (!b.splits) return 0;
     return round256(gemm_workspace_bytes(batch, m)) +
            (b.splits > 1 ? (size_t)b.splits * batch * n * 4 : 0);
+  }
   return round256(n * m * 2) + round256(n * 4) +
          (q8_0_use_stream(n, m, batch) ? f16_gemm_stream_workspace_bytes(batch, n, m, num_cus)
                                        : f16_gemm_v2_workspace_bytes(batch, n, m, num_cus));
 }
 
 hipError_t launch_q8_0_gemm(float* y, const uint8_t* w, const float* x, const float* bias,
-                            size_t n, size_t m, size_t batch, void* ws, int num_cus,
+                            size_t n, size_t m, size_t batch, void* ws, int num_cus, bool expand,
                             hipStream_t s) {
   uint8_t* base = static_cast<uint8_t*>(ws);
-  const BlockPlan b = q8_0_plan(w, n, m, batch, num_cus);
-  if (b.splits) {
+  if (!expand) {
+    const BlockPlan b = q8_0_plan(w, n, m, batch, num_cus);
     hipError_t be = launch_x_f16_onepass(x, batch, m, ws, false, s);
     if (be != hipSuccess) return be;
     return launch_block_gemm_f16x(

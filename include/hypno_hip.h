@@ -69,7 +69,13 @@
  *     from several threads on one stream are serialised for the span of
  *     their launches (each stream has its own workspace); a call needing a
  *     larger workspace than its stream holds synchronises that stream first,
- *     so make the first call of each size before capturing a HIP graph.
+ *     so make the first call of each size before capturing a HIP graph.  Where
+ *     a workspace cannot be had (device memory is full, or the stream is under
+ *     capture and holds less), the calls that have kernels without one run
+ *     those, slower and with other roundings: Q4_0 and Q8_0 batches on rows
+ *     that suit none of the tuned kernels, FP16 rows of m % 64 == 32 and
+ *     column-major batches token by token, Q4_0 of m % 64 == 0 and Q8_0 from
+ *     16 tokens on a smaller workspace.  The others are ENOMEM or EDEVICE.
  */
 #ifndef HYPNO_HIP_H
 #define HYPNO_HIP_H

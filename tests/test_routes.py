@@ -70,3 +70,25 @@ def test_q4_0_prompt_tiles(calls, tokens, n, m, block):
     got = _kernels(calls(["q4_0", n, m, tokens])[0])
     assert ("gemm_block_kernel<0,8,0,1>" in got) == block, got
     assert any(k.startswith("q4_0_gemm_exact_kernel") for k in got) == (not block), got
+
+
+# Calls that ran without a workspace, or with a smaller one, before the GEMMs that
+# want one: with no device memory left, and under capture on a stream that holds
+# too little, they still run.
+@pytest.mark.parametrize("call,room,plain", [
+    (["q4_0", 2400, 2080, 17], 0, "gemv_any_kernel<0,64>"),
+    (["q8_0", 2880, 7200, 33], 0, "gemv_any_kernel<1,64>"),
+    (["f16", 2880, 7200, 64], 0, "f16_gemv_fast_kernel"),
+    # (the tile kernel's fp16 rows; the expanded fp16 weights and activations)
+    (["q4_0", 640, 2880, 16], 128 * 2880 * 2 + 512, "gemm_kernel"),
+    (["q8_0", 255, 8192, 127], 255 * 8192 * 2 + 128 * 8192 * 2 + (2 << 20), "f16_gemm")])
+def test_no_room_for_a_workspace(calls, call, room, plain):
+    full, first = calls(["room", room], call)[1], calls(call)[0]
+    assert any(plain in k for k in _kernels(full)), full
+    assert not any(plain in k for k in _kernels(first)), first
+    # under capture, the stream holding what that plain run left
+    steps = [["room", room], call, ["room", None], ["capture", 1], call, ["capture", 0], call]
+    *_, captured, _, after = calls(*steps)
+    assert any(plain in k for k in _kernels(captured)), captured
+    assert not any(line.startswith(("malloc", "free")) for line in captured[1])
+    assert _kernels(after) == _kernels(first)
