@@ -112,10 +112,14 @@ hipError_t upload(void* dst, const void* src, size_t bytes, DevBuf& pin, hipStre
 // through the last launch of a call, so two threads calling on one stream
 // neither free a buffer the other is about to launch with nor interleave
 // their multi-kernel sequences (pre-pass, GEMM, reduction); a buffer is only
-// replaced after the stream has drained.
+// replaced after the stream has drained.  A buffer that went into a graph under
+// capture is never freed, as the graph keeps its address; the one that takes its
+// place is at least twice as large (if device memory has that much left), so all
+// that is kept is no larger than the buffer in use.
 struct StreamWs {
   std::mutex mu;
   DevBuf buf;
+  bool captured = false;  // `buf` is in some captured graph
 };
 
 struct DeviceState {
@@ -194,8 +198,17 @@ hipError_t grow_workspace(DeviceState* ds, hipStream_t s, size_t bytes, WsLock& 
   out.lk = std::unique_lock<std::mutex>(w->mu);
   if (optional && !(w->buf.p && w->buf.cap >= bytes) && is_capturing(s))
     return hipErrorStreamCaptureUnsupported;
+  if (w->captured && w->buf.cap < bytes && !is_capturing(s)) {
+    DevBuf next;
+    hipError_t e = ensure(next, std::max(bytes, 2 * w->buf.cap), s);
+    if (e == hipErrorOutOfMemory) e = ensure(next, bytes, s);
+    if (e != hipSuccess) return e;
+    w->buf = next;
+    w->captured = false;
+  }
   hipError_t e = ensure(w->buf, bytes, s);
   if (e != hipSuccess) return e;
+  if (!w->captured) w->captured = is_capturing(s);
   out.p = w->buf.p;
   return hipSuccess;
 }

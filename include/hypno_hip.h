@@ -76,6 +76,11 @@
  *     that suit none of the tuned kernels, FP16 rows of m % 64 == 32 and
  *     column-major batches token by token, Q4_0 of m % 64 == 0 and Q8_0 from
  *     16 tokens on a smaller workspace.  The others are ENOMEM or EDEVICE.
+ *     A workspace that a captured graph uses is kept until the process ends,
+ *     so a later larger call leaves the graph valid (the stream's next
+ *     workspace is at least twice as large: what is kept so is no larger than
+ *     the one in use).  Replays use the workspace of the stream that was
+ *     captured: order them against that stream's other calls.
  */
 #ifndef HYPNO_HIP_H
 #define HYPNO_HIP_H

@@ -148,3 +148,39 @@ def test_any_length_gemv_error(orc, dt, n, m, bound):
     got = _run(_lib.load(), torch, dt, wb, x, np.zeros(n, np.float32), n, m, 1, 0)
     f64 = orc.matmul_q4_0_f64 if dt == "q4_0" else orc.matmul_q8_0_f64
     assert orc.rel_l2(got[0], f64(wb, x[0], None, n, m)) <= bound
+
+
+@pytest.mark.gpu
+def test_any_shape_graph_outlives_larger_calls(orc):
+    """A captured ragged batch replays right after calls that need a larger
+    workspace on its stream."""
+    import torch
+
+    import hypno_amd as hk
+    n, m, tokens = 2400, 2080, 17
+    rng = np.random.default_rng(6)
+    wb = orc.quantize_q4_0((rng.standard_normal(n * m) * 0.02).astype(np.float32))
+    x = torch.from_numpy(rng.standard_normal((700, m)).astype(np.float32)).cuda()
+    w = torch.from_numpy(wb).cuda()
+    y, big = torch.zeros(tokens, n, device="cuda"), torch.zeros(700, n, device="cuda")
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        hk.batch_matmul(y, w, hk.DType.Q4_0, x[:tokens], n, m, tokens)
+    s.synchronize()
+    want = y.clone()
+    with torch.cuda.graph(g, stream=s):
+        hk.batch_matmul(y, w, hk.DType.Q4_0, x[:tokens], n, m, tokens)
+    for rows in (300, 700):
+        with torch.cuda.stream(s):
+            hk.batch_matmul(big[:rows], w, hk.DType.Q4_0, x[:rows], n, m, rows)
+        s.synchronize()
+        scratch = torch.full((1 << 24,), float("nan"), device="cuda")  # over freed memory
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+        del scratch
+    for t in range(tokens):
+        ref = orc.matmul_q4_0_f64(wb, x[t].cpu().numpy(), None, n, m)
+        assert orc.normwise_err(want[t].cpu().numpy(), ref) <= 2e-5

@@ -92,3 +92,18 @@ def test_no_room_for_a_workspace(calls, call, room, plain):
     assert any(plain in k for k in _kernels(captured)), captured
     assert not any(line.startswith(("malloc", "free")) for line in captured[1])
     assert _kernels(after) == _kernels(first)
+
+
+def test_captured_workspace_is_kept(calls):
+    """A workspace that went into a captured graph is not freed by a larger call;
+    one that did not is, and each next one is at least twice as large as a kept
+    one."""
+    small, large, largest = (["q4_0", 2400, 2080, t] for t in (17, 300, 700))
+    res = calls(small, ["capture", 1], small, ["capture", 0], large, largest)
+    logs = [r[1] for r in res if r]
+    assert all(r[0] == 0 for r in res if r)
+    sizes = [[int(x.split()[1]) for x in log if x.startswith("malloc")] for log in logs]
+    freed = [[int(x.split()[1]) for x in log if x.startswith("free")] for log in logs]
+    assert [len(s) for s in sizes] == [1, 0, 1, 1]
+    assert freed == [[], [], [], sizes[2]]
+    assert sizes[2][0] >= 2 * sizes[0][0]
