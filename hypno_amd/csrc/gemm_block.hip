@@ -616,8 +616,11 @@ BlockPlan block_plan(size_t n, size_t m, size_t batch, int num_cus) {
   const size_t steps = rup(m, kBStageK) / kBStageK;
   BlockPlan best{1, 1, 0.0};
   double best_cost = 1e300;
+  // (rows of an even number of blocks come with fewer than 16 tokens, or with
+  // more than the prefill kernels' limits allow: 32-row tiles only)
+  const bool odd = m / kBlockElems % 2 != 0;
   for (int mt : {1, 2}) {
-    if (mt > 1 && (size_t)16 * mt >= batch) break;  // taller tiles than the rows
+    if (mt > 1 && (!odd || (size_t)16 * mt >= batch)) break;  // taller tiles than the rows
     const size_t tm = (batch + 32 * mt - 1) / (32 * mt);
     const size_t tiles = tm * tn;
     const double stage_us = mt == 2 ? 1.2 : 0.95;
@@ -712,7 +715,8 @@ static hipError_t launch_block_mt(const BlockPlan& p, const BlockArgs& a, hipStr
     hipLaunchKernelGGL(kernel, dim3(a.tiles_m * a.tiles_n, p.splits), dim3(kBThreads), lds, s, a);
     return hipGetLastError();
   };
-  if (p.mt == 2) return go(gemm_block_kernel<FMT, 2, ODD, 3>, BlockGeom<FMT, 2, ODD>::kLds);
+  if constexpr (ODD)
+    if (p.mt == 2) return go(gemm_block_kernel<FMT, 2, ODD, 3>, BlockGeom<FMT, 2, ODD>::kLds);
   return go(gemm_block_kernel<FMT, 1, ODD, 3>, BlockGeom<FMT, 1, ODD>::kLds);
 }
 

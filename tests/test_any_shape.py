@@ -3,7 +3,8 @@ through the any-length GEMV, batches through the fp32-accurate block GEMM (and,
 for Q4_0 from 16 tokens at K % 64 == 0, the prefill GEMM).  The cases sit at
 the edges of their tiles: odd numbers of blocks per row (rows on 2-byte
 boundaries), buffers that end with the last row, x off a 16-byte boundary, one
-row or column past a tile, K pieces, lanes shared by several short rows."""
+row or column past a tile, K pieces, lanes shared by several short rows.  (test_routes.py checks which kernel
+each case runs.)"""
 import ctypes
 
 import numpy as np
@@ -16,11 +17,18 @@ CASES = [  # dtype, tokens, n, m
         # the any-length GEMV: 8, 16, 32 and 64 lanes per row
         (1, 1, 32), (1, 33, 96), (1, 257, 288), (1, 31, 544), (1, 100, 1056), (1, 65, 11008),
         (1, 7, 32768), (1, 5, 32800), (2, 97, 1120), (7, 513, 4128), (33, 257, 2080),
-        # the block GEMM: 32-, 64- and 128-row tiles, one row or column past them
-        (5, 4097, 4128), (16, 1300, 4128), (33, 1030, 2400), (64, 520, 2464), (65, 1290, 1120),
-        (129, 600, 1120), (300, 257, 1120),
-        # whole 64-column stages, from 16 tokens the prefill GEMM (Q4_0)
-        (16, 640, 2880), (17, 129, 4160)]
+        # too few products or a buffer that ends inside a dword: token by token
+        (5, 4097, 4128), (300, 257, 1120),
+        # the block GEMM, odd numbers of blocks per row, 32-row tiles, a row or column
+        # past them, one and several K pieces
+        (16, 1300, 4128), (33, 1030, 2400), (64, 520, 2464), (65, 1290, 1120),
+        (129, 600, 1120), (129, 8194, 96),
+        # 64-row tiles, one and several K pieces
+        (100, 16480, 96), (33, 11086, 736),
+        # whole 64-column stages: the block GEMM on even numbers of blocks below 16
+        # tokens, from 16 the prefill GEMMs
+        (8, 7200, 1472), (15, 4162, 1344), (2, 16000, 2880), (15, 33000, 192), (16, 640, 2880),
+        (17, 129, 4160)]
 ]
 
 

@@ -19,9 +19,11 @@ CASES = [  # dtype, tokens, n, m
     ("q8_0", 16, 257, 64), ("q8_0", 17, 33, 128), ("q8_0", 33, 4096, 4096),
     ("q8_0", 64, 300, 2048), ("q8_0", 65, 1000, 320), ("q8_0", 127, 255, 8192),
     ("q8_0", 129, 513, 1088), ("q8_0", 257, 7201, 576), ("q8_0", 1025, 8193, 256),
-    ("q8_0", 700, 1, 192), ("q8_0", 300, 1200, 16448),
+    ("q8_0", 700, 1, 192), ("q8_0", 300, 1200, 16448), ("q8_0", 300, 16385, 512),
+    ("q8_0", 128, 4097, 4160),
     ("q4_0", 1793, 5569, 1024), ("q4_0", 2048, 14336, 320), ("q4_0", 1025, 16385, 512),
-    ("q4_0", 500, 14300, 2048), ("q4_0", 512, 14336, 64),
+    ("q4_0", 500, 14300, 2048), ("q4_0", 512, 14336, 64), ("q4_0", 1024, 16383, 64),
+    ("q4_0", 2892, 2944, 3712),
 ]
 
 
@@ -80,11 +82,20 @@ def test_block_f16x(dt, tokens, n, m, shift):
     assert not bad.any(), (bad.nonzero()[:4].tolist(), (got - ref).abs().max().item())
 
 
-def test_q8_0_odd_address():
+@pytest.mark.parametrize("tokens,n,m", [(40, 129, 320), (64, 300, 1088), (130, 300, 1088),
+                                        (300, 5000, 1088)])
+def test_q8_0_odd_address(tokens, n, m):
+    """Weights at an odd 2-byte address: expanded to fp16, row by row scaled so
+    that a block scale of 60000 (weights up to 127 * 60000) stays in range, on the
+    streaming fp16 GEMM up to 64 tokens and the DMA-fed one beyond."""
     import torch
-    n, m, tokens = 129, 320, 40
     gen = torch.Generator(device="cuda").manual_seed(3)
     w, wv = _blocks(torch, gen, n, m, "q8_0")
+    big = torch.tensor([60000.0], dtype=torch.float16, device="cuda")
+    blocks = w.view(n, m // 32, 34)
+    for r, b in ((0, 0), (n - 1, m // 32 - 1)):
+        blocks[r, b, :2] = big.view(torch.uint8)
+        wv[r, 32 * b:32 * b + 32] = (blocks[r, b, 2:].double() - 128) * 60000.0
     buf = torch.empty(w.numel() + 2, dtype=torch.uint8, device="cuda")
     buf[2:] = w
     x = torch.randn(tokens, m, generator=gen, device="cuda")
@@ -92,4 +103,6 @@ def test_q8_0_odd_address():
     got = _run(torch, "q8_0", buf[2:], x, bias, n, m, tokens).double()
     ref = x.double() @ wv.t()
     # x and the weights each rounded to fp16 once: 2^-12 at random each
-    assert ((got - ref).norm() / ref.norm()).item() <= 1e-3
+    for rows in (slice(1, n - 1), slice(0, 1), slice(n - 1, n)):
+        g, r = got[:, rows], ref[:, rows]
+        assert ((g - r).norm() / r.norm()).item() <= 1e-3

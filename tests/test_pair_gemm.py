@@ -1,7 +1,8 @@
 """Batches on the pair GEMM: column-major Q4_0 at many tokens and fp16
 weights whose rows are no multiple of 64, at the edges of its tiles (row tiles
-of 32, 64 and 128 tokens, 256 output columns, 64-column stages cut in half),
-with short buffers, scales past fp16's products, infinities and biases."""
+of 32 and 64 tokens, 256 output columns, 64-column stages cut in half), with
+short buffers, scales past fp16's products, infinities and biases.
+(test_routes.py checks which kernel each case runs.)"""
 import ctypes
 
 import numpy as np
@@ -28,12 +29,18 @@ def _col(torch, wb, x, bias, n, m):
     return y.cpu().numpy()
 
 
+COL_CASES = [  # tokens, n, m, bytes cut off the end
+    (40, 2080, 2080, 0), (33, 3104, 1056, 0), (65, 1056, 1120, 0), (128, 256, 2048, 0),
+    (300, 544, 1056, 0), (64, 1056, 1056, 18 * 33 * 100 + 7), (8, 5664, 2080, 0),
+    (300, 14336, 544, 18 * 448 * 3),
+    # 64-row tiles, one and several K pieces
+    (100, 16480, 96, 0), (35, 11584, 928, 0), (100, 5632, 1056, 18 * 176 * 20),
+    # an odd number of blocks that ends the buffer: one token at a time
+    (129, 1024, 1024, 18)]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("tokens,n,m,cut", [(40, 2080, 2080, 0), (33, 3104, 1056, 0),
-                                            (65, 1056, 1120, 0), (129, 1024, 1024, 18),
-                                            (128, 256, 2048, 0), (300, 544, 1056, 0),
-                                            (64, 1056, 1056, 18 * 33 * 100 + 7),
-                                            (8, 5664, 2080, 0), (300, 14336, 544, 18 * 448 * 3)])
+@pytest.mark.parametrize("tokens,n,m,cut", COL_CASES)
 def test_col_major_many_tokens(orc, tokens, n, m, cut):
     import torch
     print(f"col tokens={tokens} n={n} m={m} cut={cut}", flush=True)
@@ -51,12 +58,13 @@ def test_col_major_many_tokens(orc, tokens, n, m, cut):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tokens,n,m", [(40, 2080, 2080), (35, 11584, 928)])
 @pytest.mark.parametrize("bits", [0x6FFF, 0x7000, 0x7BFF, 0x0001, 0x8200])
-def test_col_major_scale_range(orc, bits):
+def test_col_major_scale_range(orc, bits, tokens, n, m):
     """One block's scale at the largest whose products fp16 holds, past it, at
-    fp16's largest value, at its smallest and at a negative subnormal."""
+    fp16's largest value, at its smallest and at a negative subnormal, on 32- and
+    64-row tiles."""
     import torch
-    tokens, n, m = 40, 2080, 2080
     rng = np.random.default_rng(bits)
     wb = orc.quantize_q4_0((rng.standard_normal(n * m) * 0.02).astype(np.float32))
     g = 777 * (n // 32) + 13
@@ -73,9 +81,9 @@ def test_col_major_scale_range(orc, bits):
 
 
 @pytest.mark.gpu
-def test_col_major_infinite_token(orc):
+@pytest.mark.parametrize("tokens,n,m", [(40, 2080, 2080), (35, 11584, 928)])
+def test_col_major_infinite_token(orc, tokens, n, m):
     import torch
-    tokens, n, m = 40, 2080, 2080
     rng = np.random.default_rng(3)
     wb = orc.quantize_q4_0((rng.standard_normal(n * m) * 0.02).astype(np.float32))
     x = rng.standard_normal((tokens, m)).astype(np.float32)
@@ -90,9 +98,13 @@ def test_col_major_infinite_token(orc):
         assert orc.normwise_err(got[t], ref[t - 8]) <= 2e-5, t
 
 
+F16_CASES = [(2, 20001, 1056), (3, 20001, 1056), (16, 2600, 992), (33, 1300, 1120),
+             (65, 257, 2400), (129, 511, 1056), (300, 300, 544), (70, 16384, 1056),
+             (100, 16480, 96), (35, 11590, 928)]  # the last two: 64-row tiles
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("tokens,n,m", [(2, 20001, 1056), (16, 2600, 992), (33, 1300, 1120),
-                                        (65, 257, 2400), (129, 511, 1056), (300, 300, 544)])
+@pytest.mark.parametrize("tokens,n,m", F16_CASES)
 def test_f16_half_stage_rows(orc, tokens, n, m):
     import torch
 

@@ -220,10 +220,11 @@ GEMM_TOL = 2e-3  # rel-L2 over all M x N (north_star: MFMA prefill, fp16 activat
 @pytest.mark.parametrize("batch,n,m", [(16, 512, 256), (64, 1000, 1024), (128, 4096, 4096),
                                        (512, 2048, 2048), (20, 3, 64)])
 def test_q8_0_gemm(torch, hk, orc, batch, n, m):
-    """M >= 16 runs the fp16 GEMM on weights expanded to fp16 (per-row
-    normalised): against the per-token fp32 reference on the unrounded x
-    (turbo.rs:334-341 semantics; the fp16 rounding of x and of the weights
-    both count against the tolerance), and the bias on the device path."""
+    """M >= 16 runs on activations rounded to fp16, here on the blocks' exact
+    integers (test_block_f16x.py has the weights expanded to fp16): against the
+    per-token fp32 reference on the unrounded x (turbo.rs:334-341 semantics; the
+    rounding of x counts against the tolerance), and the bias on the device
+    path."""
     print(f"q8_0 gemm batch={batch} n={n} m={m}", flush=True)
     wq = _q8(orc, batch + n + m, n, m)
     x = orc.normal_f32(batch * 7 + m, batch * m, 1.0).reshape(batch, m)
@@ -244,8 +245,7 @@ def test_q8_0_gemm(torch, hk, orc, batch, n, m):
     got = y.cpu().numpy().reshape(batch, n)
     err = orc.rel_l2(got, ref)
     assert err <= GEMM_TOL, f"rel L2 {err:.3e}"
-    # a weight row with one huge block scale: per-row normalisation keeps the
-    # fp16 expansion finite (|w| up to 127 * 60000 > fp16 max)
+    # a weight row with one huge block scale (|w| up to 127 * 60000 > fp16 max)
     if (batch, n, m) == (16, 512, 256):
         big = wq.copy().reshape(-1, 34)
         big[0, 0:2] = np.frombuffer(np.float16(60000.0).tobytes(), np.uint8)

@@ -107,3 +107,36 @@ def test_captured_workspace_is_kept(calls):
     assert [len(s) for s in sizes] == [1, 0, 1, 1]
     assert freed == [[], [], [], sizes[2]]
     assert sizes[2][0] >= 2 * sizes[0][0]
+
+
+def _all_kernels(calls, steps):
+    return {k for r in calls(*steps) for k in _kernels(r)}
+
+
+def test_cases_reach_every_instantiation(calls):
+    """The GPU tests' lists of shapes run every instantiation of the kernels that
+    they are there for."""
+    import test_any_shape
+    import test_block_f16x
+    import test_pair_gemm
+    got = _all_kernels(calls, [[dt, n, m, t] for dt, t, n, m in test_any_shape.CASES])
+    assert {k for k in got if k.startswith(("gemm_block", "gemv_any"))} >= {
+        *(f"gemm_block_kernel<{f},{mt},{odd},3>" for f in (0, 1)
+          for mt, odd in ((1, 0), (1, 1), (2, 1))),
+        *(f"gemv_any_kernel<{f},{lanes}>" for f in (0, 1) for lanes in (8, 16, 32, 64))}
+    assert "block_split_reduce_kernel" in got
+    got = _all_kernels(calls, [[dt, n, m, t] for dt, t, n, m in test_block_f16x.CASES])
+    assert {k for k in got if k.startswith("gemm_block")} == {
+        *(f"gemm_block_kernel<1,{mt},0,1>" for mt in (2, 4, 8)), "gemm_block_kernel<0,8,0,1>"}
+    odd = [["q8_0", n, m, t, {"w_off": 2}] for t, n, m in
+           ((40, 129, 320), (64, 300, 1088), (130, 300, 1088), (300, 5000, 1088))]
+    got = [_kernels(r) for r in calls(*odd)]
+    assert all(k[0] == "q8_0_rows_to_f16_kernel" for k in got)
+    assert [any("stream" in x for x in k) for k in got] == [True, True, False, False]
+    for cases, kind, col in ((test_pair_gemm.COL_CASES, "q4_0_col", 1),
+                             (test_pair_gemm.F16_CASES, "f16", 0)):
+        got = calls(*([kind, c[1], c[2], c[0], {"extra": -c[3] if col else 0}] for c in cases))
+        tiles = [[f"gemm_pair_kernel<{mt},{col}>" in _kernels(r) for mt in (1, 2)] for r in got]
+        split = ["block_split_reduce_kernel" in _kernels(r) for r in got]
+        assert {(t[1], s) for t, s in zip(tiles, split) if any(t)} == {
+            (False, False), (False, True), (True, False), (True, True)}
