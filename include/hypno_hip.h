@@ -23,18 +23,21 @@
  *         value), products with the nibbles are exact in int32, each block's
  *         sum is scaled by d in fp32 and blocks accumulate in fp32.  Other
  *         shapes: fp32 FMAs.  Bar: max|y - r| / max|r| <= 1e-4.
- *       Q4_0 and Q8_0 batches whose rows suit none of the kernels below
- *         (m % 32 == 0): each activation as three bf16 parts that hold all its
- *         24 bits, exact products with the integers on MFMA, block scale in
- *         fp32, from 80M products; fewer take fp32 FMAs token by token.
- *       Q4_0, M = 2 (M <= 4 when n * m <= 16M),
- *         m % 256 == 0: the
+ *       Q4_0 and Q8_0 batches on rows that suit none of the kernels below
+ *         (m % 32 == 0; below 16 tokens m % 256 != 0 or x not 16-byte aligned,
+ *         from 16 tokens m % 64 == 32): each activation as three bf16 parts
+ *         that hold all its 24 bits, exact products with the integers on MFMA,
+ *         block scale in fp32; the 1e-4 bar per token.  From 80M products;
+ *         fewer, and a weight buffer that ends with its last row at 2 mod 4
+ *         bytes (n * m / 32 odd), take fp32 FMAs token by token.
+ *       Q4_0, M = 2 (M = 3 when n * m <= 16M), m % 256 == 0: the
  *         streaming GEMV with every block multiplied by each token's row, in
  *         its arithmetic above (each token's y bit-identical to its M = 1
- *         result).  Otherwise M = 2..16: fp16 hi/lo activation pairs per
- *         256-column stage (to ~2^-22), exact nibble products on MFMA, fp32
- *         block scale; the same 1e-4 bar per token.
- *       Q4_0, M = 17..64, and M >= 65 (prefill GEMM): activations rounded to
+ *         result).  Otherwise M = 2..16, m % 256 == 0: fp16 hi/lo activation
+ *         pairs per 256-column stage (to ~2^-22), exact nibble products on
+ *         MFMA, fp32 block scale; the same 1e-4 bar per token.
+ *       Q4_0, M = 17..64 (M = 16 too where m % 64 == 0 but m % 256 != 0), and
+ *         M >= 65 (prefill GEMM), m % 64 == 0: activations rounded to
  *         fp16 after a power-of-two scale per token (undone exactly on the
  *         output), fp32 accumulation on MFMA.  Weights: the exact integer
  *         nibbles (fp16 -8..7), each block's d applied to its partial sum in
@@ -46,15 +49,15 @@
  *         ||Y - R||_2 / ||R||_2 <= 2e-3.
  *       FP16: M = 1 fp32 FMAs; M = 2..15 each token as two fp16 rows, hi and
  *         lo (x 2^s = hi + lo to ~2^-22), on MFMA against the fp16 weights
- *         with fp32 accumulation (the 1e-4 bar per token; fp32 FMAs token by
- *         token if x is not 16-byte aligned); M >= 16 as the Q4_0 GEMM with
- *         fp16 weights.  Rows of m % 64 == 32: from 3 tokens (3 from
- *         17M products on) activations in three bf16 parts and weights in two,
- *         both exact, on MFMA with fp32 accumulation; fewer fp32 FMAs token
- *         by token.
- *       Q8_0: M < 16 each token's activations as three exact int8 digit
- *         planes per block (to 2^-23), each weight block read once for 2 to 8
- *         tokens; M >= 16 as the Q4_0 GEMM with exact integer weights, or
+ *         with fp32 accumulation (the 1e-4 bar per token); M >= 16 as the Q4_0
+ *         GEMM with fp16 weights; both m % 64 == 0.  Rows of m % 64 == 32, and
+ *         M < 16 where x is not 16-byte aligned (m % 32 == 0): from 4 tokens,
+ *         or 3 from 17M products on, activations in three bf16 parts and
+ *         weights in two, both exact, on MFMA with fp32 accumulation (the same
+ *         bar).  All other FP16 calls: fp32 FMAs token by token.
+ *       Q8_0: M < 16, m % 256 == 0, each token's activations as three exact
+ *         int8 digit planes per block (to 2^-23), each weight block read once
+ *         for 2 to 8 tokens; M >= 16, m % 64 == 0, as the Q4_0 GEMM with exact integer weights, or
  *         where that is faster weights expanded once to fp16
  *         (row-normalised, relative 2^-11) and the FP16 GEMM.
  *       Column-major Q4_0: fp32 FMAs token by token; from 8 tokens, where it
@@ -236,10 +239,11 @@ int hypno_hip_matmul_f16_dev(float* y, const uint8_t* w, size_t w_len, const flo
 /* Q8_0 on device pointers (ops.rs:33-36 for batch == 1; turbo.rs:334-341
  * semantics for batch > 1).  batch >= 16 with m % 64 == 0 runs a prefill
  * GEMM on the blocks or on an fp16 expansion of the weights, whichever a cost
- * model has faster (rel-L2 <= 2e-3 of the exact product); smaller batches (m % 256 == 0, x 16-byte aligned) read each
- * weight block once per 2 to 8 tokens, every token's row bit-identical to
- * its one-token call (normwise <= 1e-4); other shapes run an fp32-accurate
- * MFMA GEMM from 80M products (m % 32 == 0), token by token below. */
+ * model has faster (rel-L2 <= 2e-3 of the exact product); smaller batches
+ * (m % 256 == 0, x 16-byte aligned) read each weight block once per 2 to 8
+ * tokens, every token's row bit-identical to its one-token call (normwise <=
+ * 1e-4); other shapes run an fp32-accurate MFMA GEMM from 80M products
+ * (m % 32 == 0), token by token below. */
 int hypno_hip_matmul_q8_0_dev(float* y, const uint8_t* w_q, size_t w_len, const float* x,
                               const float* bias, size_t n, size_t m, size_t batch,
                               void* stream);
